@@ -123,6 +123,11 @@ struct Level {
     // FP32 copies for the mixed-precision V-cycle (allocated on first use):
     // w (level 0: of ctx->w; wf2 of ctx->w22 when K is anisotropic), x, b, r
     float *wf, *wf2, *xf, *bf, *rf;
+    // the assembled 9-point operator (nu < 1, allocated on first use): ten
+    // planes of plane9 doubles, pitch ld9 (OpPlanes)
+    double *a9;
+    long plane9;
+    int ld9;
 };
 
 struct ProfEntry {
@@ -166,6 +171,7 @@ struct impec_ctx {
     // correction since the last reliable update, direction pair, matvec, and
     // FP32 copies of fx / fy
     float *pr32, *pe32, *pd32, *pz32, *pq32, *fx32, *fy32;
+    double *op9_inv;           // coarsest level's solution operator of the 9-point cycle
     double *scal;              // device scalars (Scal)
     double *part;              // reduction partials
     double *part_mid;          // per-thread shares of a two-stage finish (FIN_THREADS x PART_VECS)

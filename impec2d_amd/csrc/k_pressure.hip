@@ -17,6 +17,7 @@
 #include <math.h>
 #include <stdlib.h>
 #include <type_traits>
+#include "mg_block.h"
 #include <vector>
 
 namespace impec {
@@ -450,6 +451,64 @@ __global__ void k_coarsest(LevArgs L, T *__restrict__ x, const T *__restrict__ b
     coarsest_body<DIAG, T>(HwGrid{}, L, x, b);
 }
 
+// the assembled 9-point operator of a level (OpPlanes): op_row's folded rows
+// and the reciprocal diagonals, formed once per solve.  A V-cycle's legs read
+// every row eight times or more; forming it costs eight divisions.
+__global__ void k_op9(LevArgs L, double *__restrict__ A, long plane, int ld) {
+    const int j = blockIdx.x * blockDim.x + threadIdx.x;
+    const int i = blockIdx.y * blockDim.y + threadIdx.y;
+    if (i >= L.g.n1 || j >= L.g.n2) return;
+    double a[9];
+    op_row<true>(L.g, L.w1, L.w2, L.ldw, i, j, a);
+    double *p = A + (long)i * ld + j;
+#pragma unroll
+    for (int k = 0; k < 9; k++) p[k * plane] = a[k];
+    p[9 * plane] = a[ST_C] != 0. ? 1. / a[ST_C] : 0.;
+}
+
+// the coarsest level's solution operator (row-major n x n): column k is the
+// solution of coarsest_solve for the k-th unit right-hand side, on thread k
+template <int N1, int N2>
+__device__ __forceinline__ void coarsest_inv(const LevArgs &L, double *__restrict__ inv, int k) {
+    constexpr int n = N1 * N2, m = n + 1;
+    const int dI[9] = {0, -1, -1, 0, 1, 1, 1, 0, -1}, dJ[9] = {0, 0, -1, -1, -1, 0, 1, 1, 1};
+    double M[m][m + 1];
+#pragma unroll
+    for (int r = 0; r < m; r++)
+#pragma unroll
+        for (int q = 0; q <= m; q++) M[r][q] = 0.;
+#pragma unroll
+    for (int i = 0; i < N1; i++)
+#pragma unroll
+        for (int j = 0; j < N2; j++) {
+            const int row = i * N2 + j;
+            double a[9];
+            op_row<true>(L.g, L.w1, L.w2, L.ldw, i, j, a);
+#pragma unroll
+            for (int q = 0; q < 9; q++) {
+                const int ii = i + dI[q], jj = j + dJ[q];
+                if (ii < 0 || jj < 0 || ii >= N1 || jj >= N2) continue;
+                M[row][ii * N2 + jj] += a[q];
+            }
+            M[row][n] = 1.;
+            M[n][row] = 1.;
+            M[row][m] = row == k ? 1. : 0.;
+        }
+    double sol[m];
+    bordered_solve<n, false>(M, sol);
+#pragma unroll
+    for (int r = 0; r < n; r++) inv[r * n + k] = sol[r];
+}
+__global__ void k_op9_coarsest(LevArgs L, double *__restrict__ inv) {
+    const int n1 = L.g.n1, n2 = L.g.n2, k = threadIdx.x;
+    if (k >= n1 * n2) return;
+    // the hierarchy is coarsened until both sides are at most 2
+    if (n1 == 2 && n2 == 2) coarsest_inv<2, 2>(L, inv, k);
+    else if (n1 == 2 && n2 == 1) coarsest_inv<2, 1>(L, inv, k);
+    else if (n1 == 1 && n2 == 2) coarsest_inv<1, 2>(L, inv, k);
+    else if (n1 == 1 && n2 == 1) coarsest_inv<1, 1>(L, inv, k);
+}
+
 // ---------------------------------------------------------------------------
 // conjugate-gradient vector kernels (level-0 ring-1 layout; x lives in p)
 // ---------------------------------------------------------------------------
@@ -879,6 +938,9 @@ static LevArgs lev_args(const impec_ctx *ctx, int l) {
 
 static int round_up(int x, int m) { return (x + m - 1) / m * m; }
 
+static bool blocks9_ok(const impec_ctx *ctx);
+static bool op9_alloc(impec_ctx *ctx);
+
 int pressure_setup_levels(impec_ctx *ctx) {
     int n1 = ctx->N1, n2 = ctx->N2;
     double dx = ctx->dx, dy = ctx->dy;
@@ -915,6 +977,7 @@ int pressure_setup_levels(impec_ctx *ctx) {
         if (hipMalloc(vecs[k], bytes0) != hipSuccess) return set_error(ctx, IMPEC_ENOMEM, "CG vector allocation failed");
         hipMemset(*vecs[k], 0, bytes0);
     }
+    if (ctx->P.nu != 1. && blocks9_ok(ctx)) op9_alloc(ctx);
     return IMPEC_OK;
 }
 
@@ -923,11 +986,14 @@ void pressure_free_levels(impec_ctx *ctx) {
         Level &L = ctx->lev[l];
         hipFree(L.x); hipFree(L.b); hipFree(L.r);
         hipFree(L.wf); hipFree(L.wf2); hipFree(L.xf); hipFree(L.bf); hipFree(L.rf);
+        if (L.a9) hipFree(L.a9);
         if (L.w) hipFree(L.w);
     }
     ctx->nlev = 0;
     hipFree(ctx->pr); hipFree(ctx->pz); hipFree(ctx->pd); hipFree(ctx->pq);
     hipFree(ctx->fx); hipFree(ctx->fy);
+    if (ctx->op9_inv) hipFree(ctx->op9_inv);
+    ctx->op9_inv = nullptr;
     float **v32[7] = {&ctx->pr32, &ctx->pe32, &ctx->pd32, &ctx->pz32, &ctx->pq32, &ctx->fx32, &ctx->fy32};
     for (float **v : v32) {
         if (*v) hipFree(*v);
@@ -2030,6 +2096,46 @@ __global__ void __launch_bounds__(64 * SW_WAVES) k_dir_mv(DirMvArgs<T, DT> A, co
     dir_mv_body<T, DT>(A, dold, dnew, first, xcd_wave());
 }
 
+// The direction update and matvec of k_dir_mv for the assembled 9-point
+// operator, one cell per thread: d_new at the cell's nine points is formed from
+// the V-cycle output and the old direction (cached: every value is read by nine
+// threads), and the cell's own is stored.
+__global__ void __launch_bounds__(256) k_dir_mv9(OpPlanes<double> A, CgArgs c, const double *__restrict__ x0,
+                                                 const double *__restrict__ dold, double *__restrict__ dnew,
+                                                 double *__restrict__ qv, const double *__restrict__ S, int first,
+                                                 double *__restrict__ part) {
+    const double mean = S[S_ZSUM] / (double)c.n;
+    const double beta = first ? 0. : S[S_RHO] / S[S_RHO_OLD];
+    const int j = blockIdx.x * 64 + threadIdx.x;
+    double s[1] = {0.};
+    for (int i = blockIdx.y * 4 + threadIdx.y; i < c.n1; i += gridDim.y * 4) {
+        if (j >= c.n2) break;
+        const long o = (long)(i + 1) * c.ld + (j + 1);
+        auto dn = [&](int di, int dj) -> double {
+            if (!c.shift && i + di == c.pin_i && j + dj == c.pin_j) return 0.;
+            const long q = o + (long)di * c.ld + dj;
+            return first ? x0[q] - mean : (x0[q] - mean) + beta * dold[q];
+        };
+        const double *a = A.a + (long)i * A.ld + j;
+        const double dc = dn(0, 0);
+        double y = a[0] * dc;
+        y += a[ST_W * A.plane] * dn(-1, 0);
+        y += a[ST_SW * A.plane] * dn(-1, -1);
+        y += a[ST_S * A.plane] * dn(0, -1);
+        y += a[ST_SE * A.plane] * dn(1, -1);
+        y += a[ST_E * A.plane] * dn(1, 0);
+        y += a[ST_NE * A.plane] * dn(1, 1);
+        y += a[ST_N * A.plane] * dn(0, 1);
+        y += a[ST_NW * A.plane] * dn(-1, 1);
+        if (!c.shift && i == c.pin_i && j == c.pin_j) y = 0.;
+        dnew[o] = dc;
+        qv[o] = y;
+        s[0] += dc * y;
+    }
+    block_reduce<RED_SUM, 1>(s);
+    if (tid_linear() == 0) part[blockIdx.y * gridDim.x + blockIdx.x] = s[0];
+}
+
 // The pinned system's true residual, streamed like k_dir_mv: a wave owns
 // DM_OUT columns (one per lane, a halo lane on each side) and a chunk of R
 // rows; it reads x and q of each row once, keeps rows i-1, i, i+1 of x in
@@ -2474,6 +2580,135 @@ static int vcycle_first_leg(impec_ctx *ctx) {
     return mg_ns(ctx) == 2 ? vcycle_first_leg_ns<T, 2>(ctx) : vcycle_first_leg_ns<T, 1>(ctx);
 }
 
+// ---- the 9-point cycle on blocks (mg_block.h) -------------------------------
+constexpr int LEG9_P = 32;   // blocks a side of a tile
+
+static OpPlanes<double> op_planes(const Level &L) { return OpPlanes<double>{L.a9, L.plane9, L.ld9}; }
+
+// first level handled by k_mg9_bottom
+static int bottom_level9(const impec_ctx *ctx) {
+    int l = 1;
+    while (ctx->lev[l].n1 > 64 || ctx->lev[l].n2 > 64) l++;
+    return l;
+}
+
+// whether the block cycle covers this problem (its own two or one sweeps per
+// leg, at least three levels, partial sums within their buffer)
+static bool blocks9_ok(const impec_ctx *ctx) {
+    if (ctx->force_unfused || ctx->nlev < 3) return false;
+    if (!((ctx->P.mg_pre <= 1 && ctx->P.mg_post <= 1) || mg_ns(ctx) == 2)) return false;
+    const Level &L = ctx->lev[0];
+    const long ti = tile_count((L.n1 + 1) / 2, LEG9_P, Halo9<1>::UI), tj = tile_count((L.n2 + 1) / 2, LEG9_P, Halo9<2>::UJ);
+    return ti * tj * 2 <= RED_BLOCKS;
+}
+
+// the planes of every level's assembled operator; false when the device has
+// no room for them (the one-kernel-per-pass cycle then runs)
+static bool op9_alloc(impec_ctx *ctx) {
+    bool ok = true;
+    for (int l = 0; ok && l < ctx->nlev; l++) {
+        Level &L = ctx->lev[l];
+        L.ld9 = round_up(L.n2, 16);
+        L.plane9 = (long)((L.n1 + 1) & ~1) * L.ld9;
+        const size_t bytes = sizeof(double) * 10 * (size_t)L.plane9;
+        ok = hipMalloc(&L.a9, bytes) == hipSuccess && hipMemset(L.a9, 0, bytes) == hipSuccess;
+    }
+    ok = ok && hipMalloc(&ctx->op9_inv, sizeof(double) * 16) == hipSuccess;
+    if (!ok) {
+        (void)hipGetLastError();
+        for (int l = 0; l < ctx->nlev; l++)
+            if (ctx->lev[l].a9) {
+                hipFree(ctx->lev[l].a9);
+                ctx->lev[l].a9 = nullptr;
+            }
+        if (ctx->op9_inv) hipFree(ctx->op9_inv);
+        ctx->op9_inv = nullptr;
+    }
+    return ok;
+}
+
+static int op9_assemble(impec_ctx *ctx) {
+    const dim3 blk(64, 4);
+    for (int l = 0; l < ctx->nlev; l++) {
+        const Level &L = ctx->lev[l];
+        hipLaunchKernelGGL(k_op9, grid2(L.n1, L.n2, blk), blk, 0, ctx->stream, lev_args(ctx, l), L.a9, L.plane9, L.ld9);
+    }
+    hipLaunchKernelGGL(k_op9_coarsest, dim3(1), dim3(64), 0, ctx->stream, lev_args(ctx, ctx->nlev - 1), ctx->op9_inv);
+    IMPEC_HIP_CHECK(ctx, hipGetLastError());
+    return IMPEC_OK;
+}
+
+static Leg9Args leg9_args(const impec_ctx *ctx, int l, int hi, int hj) {
+    Leg9Args A;
+    memset(&A, 0, sizeof(A));
+    const Level &L = ctx->lev[l], &C = ctx->lev[l + 1];
+    A.A = op_planes(L);
+    A.n1 = L.n1; A.n2 = L.n2; A.ld = L.ld;
+    A.b = (l == 0 ? ctx->pr : L.b) + L.ld + 1;
+    A.S = ctx->scal;
+    A.inv_n = 1.0 / ((double)ctx->N1 * ctx->N2);
+    A.x = L.x + L.ld + 1;
+    A.xo = L.r + L.ld + 1;
+    A.bc = C.b + C.ld + 1;
+    A.xc = C.r + C.ld + 1;
+    A.m1 = C.n1; A.m2 = C.n2; A.ldc = C.ld;
+    A.ti = tile_count((L.n1 + 1) / 2, LEG9_P, hi);
+    A.tj = tile_count((L.n2 + 1) / 2, LEG9_P, hj);
+    A.part = ctx->part;
+    return A;
+}
+
+static Bot9Args bot9_args(const impec_ctx *ctx, int lb) {
+    Bot9Args A;
+    memset(&A, 0, sizeof(A));
+    const Level &B = ctx->lev[lb];
+    const int s = B.n1 > B.n2 ? B.n1 : B.n2;
+    A.d0 = 0;
+    while (A.d0 < 4 && s <= (64 >> (A.d0 + 1))) A.d0++;
+    A.nl = ctx->nlev - lb;
+    for (int l = lb; l < ctx->nlev; l++) {
+        A.lev[l - lb].A = op_planes(ctx->lev[l]);
+        A.lev[l - lb].n1 = ctx->lev[l].n1;
+        A.lev[l - lb].n2 = ctx->lev[l].n2;
+    }
+    A.inv = ctx->op9_inv;
+    A.b = B.b + B.ld + 1;
+    A.out = B.r + B.ld + 1;
+    A.ldb = A.ldo = B.ld;
+    return A;
+}
+
+// one cycle on r - mean(r): two launches per level down to the bottom, which is
+// one; the result is left in lev[0].r, with per-tile partials for k_finish_rho
+// (*parts of them)
+template <int NS>
+static int vcycle9(impec_ctx *ctx, int *parts) {
+    using H = Halo9<NS>;
+    const int lb = bottom_level9(ctx);
+    const dim3 blk(LEG9_P * LEG9_P);
+    for (int l = 0; l < lb; l++) {
+        const Leg9Args A = leg9_args(ctx, l, H::DI, H::DJ);
+        prof_begin(ctx);
+        if (l == 0) hipLaunchKernelGGL((k_mg9_down<LEG9_P, NS, true>), dim3(A.ti * A.tj), blk, 0, ctx->stream, A);
+        else hipLaunchKernelGGL((k_mg9_down<LEG9_P, NS, false>), dim3(A.ti * A.tj), blk, 0, ctx->stream, A);
+        prof_end(ctx, l == 0 ? "mg_down_l0" : "mg_coarse");
+    }
+    const Bot9Args B = bot9_args(ctx, lb);
+    prof_begin(ctx);
+    hipLaunchKernelGGL((k_mg9_bottom<NS>), dim3(1), dim3(B.d0 == 0 ? 1024 : 256), 0, ctx->stream, B);
+    prof_end(ctx, "mg_coarse");
+    for (int l = lb - 1; l >= 0; l--) {
+        const Leg9Args A = leg9_args(ctx, l, H::UI, H::UJ);
+        prof_begin(ctx);
+        if (l == 0) hipLaunchKernelGGL((k_mg9_up<LEG9_P, NS, true>), dim3(A.ti * A.tj), blk, 0, ctx->stream, A);
+        else hipLaunchKernelGGL((k_mg9_up<LEG9_P, NS, false>), dim3(A.ti * A.tj), blk, 0, ctx->stream, A);
+        prof_end(ctx, l == 0 ? "mg_up_l0" : "mg_coarse");
+        *parts = A.ti * A.tj;
+    }
+    IMPEC_HIP_CHECK(ctx, hipGetLastError());
+    return IMPEC_OK;
+}
+
 // FP32 copy of a mobility array (rows x cols cells from (0,0) of each)
 template <class G>
 __device__ __forceinline__ void to_f32_body(const G &gr_, const double *__restrict__ src, int lds, float *__restrict__ dst, int ldd, int rows,
@@ -2661,6 +2896,30 @@ static int cg_iteration_fused(impec_ctx *ctx, const LevArgs &a0, const CgArgs &c
     return IMPEC_OK;
 }
 
+// one CG iteration with the block cycle of the 9-point operator; d ping-pongs
+static int cg_iteration_blocks9(impec_ctx *ctx, const CgArgs &c, bool first, double **dold, double **dnew) {
+    const Level &L0 = ctx->lev[0];
+    hipStream_t s = ctx->stream;
+    const Grid2 vg = vec_grid(ctx->N1, ctx->N2);
+    int st, parts = 0;
+    if ((st = mg_ns(ctx) == 2 ? vcycle9<2>(ctx, &parts) : vcycle9<1>(ctx, &parts))) return st;
+    hipLaunchKernelGGL(k_finish_rho, dim3(1), dim3(1024), 0, s, ctx->part, parts, 1.0 / (double)c.n, ctx->scal);
+    prof_begin(ctx);
+    hipLaunchKernelGGL(k_dir_mv9, vg.grid, vg.block, 0, s, op_planes(L0), c, L0.r, *dold, *dnew, ctx->pq, ctx->scal,
+                       first ? 1 : 0, ctx->part);
+    prof_end(ctx, "cg_dir_matvec");
+    if ((st = finish_sum(ctx, vg.nblocks, 1, S_DQ))) return st;
+    prof_begin(ctx);
+    hipLaunchKernelGGL(k_cg_update2, vg.grid, vg.block, 0, s, c, ctx->p, *dnew, ctx->pr, ctx->pq, ctx->scal, ctx->part);
+    prof_end(ctx, "cg_update");
+    if ((st = finish_sum(ctx, vg.nblocks, 2, S_RR, pub_next(ctx)))) return st;
+    IMPEC_HIP_CHECK(ctx, hipGetLastError());
+    double *t = *dold;
+    *dold = *dnew;
+    *dnew = t;
+    return IMPEC_OK;
+}
+
 // one iteration of the FP32-vector CG (IMPEC_PREC_MIXED32): the FP32 V-cycle
 // on the FP32 residual, the FP32 direction and matvec (FP32 faces), the FP32
 // updates of the residual and of the correction accumulated since the last
@@ -2749,6 +3008,7 @@ static int solve_cg(impec_ctx *ctx, int *its_out, double *relres_out) {
     st = build_hierarchy(ctx, F32);
     if (st) return st;
     if (F32 && (st = mixed_convert(ctx, 1))) return st;
+    if (DIAG && FUSED && (st = op9_assemble(ctx))) return st;
     // the FP32-vector CG with reliable FP64 updates (streaming 5-point path)
     const bool m32 = std::is_same<T, float>::value && FUSED && !DIAG && ctx->P.precision == IMPEC_PREC_MIXED32;
     const Level &L0 = ctx->lev[0];
@@ -2880,12 +3140,13 @@ static int solve_cg(impec_ctx *ctx, int *its_out, double *relres_out) {
                 // last reduction; the unfused one is published separately
                 if (ru) st = cg_iteration_mixed32(ctx, a0, c, since == 0, &dold32, &dnew32);
                 else if (FUSED && !DIAG) st = cg_iteration_fused<T>(ctx, a0, c, since == 0, &dold, &dnew, leg_queued);
+                else if (FUSED) st = cg_iteration_blocks9(ctx, c, since == 0, &dold, &dnew);
                 else st = cg_iteration_unfused<DIAG>(ctx, a0, c, nb, since == 0);
                 if (st) return st;
                 const bool ahead = lookahead && rr > ctx->cg_ahead * (tol * tol * bb);
                 if (ahead && (st = vcycle_first_leg<T>(ctx))) return st;
                 leg_queued = ahead;
-                if ((st = (ru || (FUSED && !DIAG)) ? wait_scalars(ctx) : fetch_scal(ctx))) return st;
+                if ((st = (ru || FUSED) ? wait_scalars(ctx) : fetch_scal(ctx))) return st;
                 its++;
                 since++;
                 // the recursion broke down (it took no step): restart it from
@@ -3012,7 +3273,8 @@ int pressure_solve(impec_ctx *ctx, int *its, double *relres) {
         IMPEC_HIP_CHECK(ctx, hipMemcpyAsync(ctx->p_prev, ctx->p, sizeof(double) * (size_t)(ctx->N1 + 2 * ctx->B) *
                                                                      ctx->lds,
                                             hipMemcpyDeviceToDevice, ctx->stream));
-    if (ctx->P.nu != 1.) return solve_cg<true, false>(ctx, its, relres);
+    if (ctx->P.nu != 1.)
+        return ctx->op9_inv ? solve_cg<true, true>(ctx, its, relres) : solve_cg<true, false>(ctx, its, relres);
     const bool fused_ok = ((ctx->P.mg_pre <= 1 && ctx->P.mg_post <= 1) || mg_ns(ctx) == 2) &&
                           fused_args<double>(ctx, 0).nwave <= RED_BLOCKS && !ctx->force_unfused;
     // mixed precision: FP32 V-cycles as the preconditioner of the FP64 CG (a
