@@ -14,10 +14,10 @@
 // the remaining rows.  Either way the returned residual is that of the
 // reference's pinned system.
 #include "impec_device.h"
+#include "mg_block.h"
 #include <math.h>
 #include <stdlib.h>
 #include <type_traits>
-#include "mg_block.h"
 #include <vector>
 
 namespace impec {
@@ -348,55 +348,6 @@ __device__ __forceinline__ void coarsen_w_body(const G &gr_, const double *__res
 __global__ void k_coarsen_w(const double *__restrict__ wf, int ldf, int n1, int n2, double *__restrict__ wc, int ldc,
                             int m1, int m2, float *__restrict__ wcf) {
     coarsen_w_body(HwGrid{}, wf, ldf, n1, n2, wc, ldc, m1, m2, wcf);
-}
-
-// Gaussian elimination with partial pivoting, then back substitution, of a
-// bordered system of n = N cells: M holds the (N+1) x (N+1) matrix and, in
-// column N+1, the right-hand side; sol receives the N+1 unknowns.  The sizes
-// are compile-time constants and every loop is unrolled, so M stays in
-// registers (with a run-time size it lives in scratch memory and each of the
-// elimination's dependent accesses is a memory round trip).  The pivot row is
-// exchanged by selects over the candidate rows, which keeps every index
-// static.  FUSED: the updates rounded once, as fused multiply-adds; otherwise
-// as a rounded product and a rounded difference.
-template <int N, bool FUSED>
-__device__ __forceinline__ void bordered_solve(double (&M)[N + 1][N + 2], double (&sol)[N + 1]) {
-    constexpr int m = N + 1;
-#pragma unroll
-    for (int col = 0; col < m; col++) {
-        int piv = col;
-        double best = fabs(M[col][col]);
-#pragma unroll
-        for (int r = col + 1; r < m; r++) {
-            const double a = fabs(M[r][col]);
-            if (a > best) { piv = r; best = a; }
-        }
-#pragma unroll
-        for (int r = col + 1; r < m; r++) {
-            const bool sw = piv == r;
-#pragma unroll
-            for (int q = 0; q <= m; q++) {
-                const double a = M[col][q], b = M[r][q];
-                M[col][q] = sw ? b : a;
-                M[r][q] = sw ? a : b;
-            }
-        }
-        const double d = M[col][col];
-        if (d == 0.) continue;
-#pragma unroll
-        for (int r = col + 1; r < m; r++) {
-            const double f = M[r][col] / d;
-#pragma unroll
-            for (int q = col; q <= m; q++) M[r][q] = FUSED ? fma(-f, M[col][q], M[r][q]) : M[r][q] - f * M[col][q];
-        }
-    }
-#pragma unroll
-    for (int r = m - 1; r >= 0; r--) {
-        double t = M[r][m];
-#pragma unroll
-        for (int q = r + 1; q < m; q++) t = FUSED ? fma(-M[r][q], sol[q], t) : t - M[r][q] * sol[q];
-        sol[r] = M[r][r] != 0. ? t / M[r][r] : 0.;
-    }
 }
 
 // coarsest level of N1 x N2 <= 2 x 2 cells: exact solve of the singular
@@ -1173,27 +1124,6 @@ struct FusedArgsT {
 };
 using FusedArgs = FusedArgsT<double>;
 
-// 1/d from the hardware reciprocal estimate refined by one Newton-Raphson
-// step, r' = r + r (1 - d r).  Only the multigrid preconditioner uses it: its
-// rounding differs from IEEE division but is the same every time for the same
-// d, so the preconditioner stays a fixed linear operator.
-__device__ __forceinline__ double recip(double d) {
-    const double r = __builtin_amdgcn_rcp(d);
-    const double e = fma(-d, r, 1.);
-    return fma(r, e, r);
-}
-__device__ __forceinline__ float recip(float d) {
-    const float r = __builtin_amdgcn_rcpf(d);
-    const float e = fmaf(-d, r, 1.f);
-    return fmaf(r, e, r);
-}
-
-// face mobility as face_mob, with recip in place of the division
-template <typename T>
-__device__ __forceinline__ T face_mob_pc(T wl, T wr, int harmonic) {
-    return harmonic ? T(2) * recip(wl + wr) : T(0.5) * (wl + wr);
-}
-
 // scaled face coefficients of one row for a lane's two columns g0, g0+1:
 // E = face to the next row, S0 = face left of g0, M = between g0 and g0+1,
 // N1 = face right of g0+1 (zero where the face is a domain boundary)
@@ -1640,286 +1570,31 @@ __global__ void __launch_bounds__(64 * SW_WAVES) k_mg_up(FusedArgsT<T> A) {
     mg_up_body<FINE0, ANISO, T, NS, R32>(A, xcd_wave());
 }
 
-// ===========================================================================
-// The bottom of the streaming V-cycle: from the first level of at most
-// BOTTOM_N x BOTTOM_N cells down to the coarsest and back up in one
-// workgroup, with every level's x, b, r, w and faces in LDS.  Per cell it does
-// what the streaming legs do (faces from w by the same expressions, red then black
-// from a zero guess, residual, full weighting; bilinear prolongation, black,
-// red), and on the coarsest level k_coarsest's bordered solve of the legs'
-// operator (faces from w, boundary faces dropped) assembled from LDS;
-// barriers separate the colour and transfer phases.  It replaces two launches
-// per small level, each a latency chain, and the one-thread coarsest launch.
-// ===========================================================================
-constexpr int BOTTOM_N = 32, BOTTOM_LEVELS = 8, BOTTOM_THREADS = 1024;
-constexpr int BOTTOM_CELLS = 1024 + 256 + 64 + 16 + 4;   // levels of at most 32, 16, 8, 4, 2 cells a side
-
-template <typename T>
-struct BottomLev {
-    const T *w;      // mobility quantity at cell (0,0), pitch ldw
-    int ldw, n1, n2, harmonic;
-    double cx, cy;
-};
-template <typename T>
-struct BottomArgs {
-    int nl;                        // levels, the last one the coarsest
-    BottomLev<T> lev[BOTTOM_LEVELS];
-    const T *b;                    // right-hand side of the first level at (0,0), pitch ldb
-    int ldb;
-    T *out;                        // its corrected, smoothed x at (0,0), pitch ldo
-    int ldo;
-    int ns;                        // red-black pairs per leg, as the streaming legs
-    const double *S;               // loop state (ensembles)
-};
-
-// the four faces of cell (i,j) of an n1 x n2 level (zero on the boundary)
-template <typename T>
-__device__ __forceinline__ void bottom_faces(const T *w, int n1, int n2, int i, int j, T cx, T cy, int harmonic,
-                                             T &W, T &E, T &Sf, T &N) {
-#pragma clang fp contract(fast)
-    const T wc = w[i * n2 + j];
-    W = i > 0 ? cx * face_mob_pc(w[(i - 1) * n2 + j], wc, harmonic) : T(0);
-    E = i < n1 - 1 ? cx * face_mob_pc(wc, w[(i + 1) * n2 + j], harmonic) : T(0);
-    Sf = j > 0 ? cy * face_mob_pc(w[i * n2 + j - 1], wc, harmonic) : T(0);
-    N = j < n2 - 1 ? cy * face_mob_pc(wc, w[i * n2 + j + 1], harmonic) : T(0);
-}
-
-// the bottom's coarsest level of N1 x N2 cells: the bordered solve of the
-// legs' operator (faces from w, boundary faces dropped), w, b and x at the
-// level's place in LDS
-template <int N1, int N2, typename T>
-__device__ __forceinline__ void bottom_coarsest(const T *w, const T *b, T *x, T cx, T cy, int hm) {
-    constexpr int n = N1 * N2, m = n + 1;
-    double M[m][m + 1];
-#pragma unroll
-    for (int r = 0; r < m; r++)
-#pragma unroll
-        for (int q = 0; q <= m; q++) M[r][q] = 0.;
-#pragma unroll
-    for (int i = 0; i < N1; i++)
-#pragma unroll
-        for (int j = 0; j < N2; j++) {
-            const int row = i * N2 + j;
-            T W, E, Sf, N;
-            bottom_faces(w, N1, N2, i, j, cx, cy, hm, W, E, Sf, N);
-            M[row][row] += (double)(-((W + E) + (Sf + N)));
-            if (i > 0) M[row][row - N2] += (double)W;
-            if (i < N1 - 1) M[row][row + N2] += (double)E;
-            if (j > 0) M[row][row - 1] += (double)Sf;
-            if (j < N2 - 1) M[row][row + 1] += (double)N;
-            M[row][n] = 1.;
-            M[n][row] = 1.;
-            M[row][m] = (double)b[row];
-        }
-    double sol[m];
-    bordered_solve<n, true>(M, sol);
-#pragma unroll
-    for (int k = 0; k < n; k++) x[k] = (T)sol[k];
-}
-
-// the faces of cell id = (i, j) of an n1 x n2 level from the per-level face
-// arrays in LDS: fw the face to row i-1, fs the face to column j-1 (each zero
-// on the boundary), so the east and north faces are the neighbours' fw and fs;
-// C the diagonal
-template <typename T>
-struct BFaces {
-    T W, E, S, N, C;
-};
-template <typename T>
-__device__ __forceinline__ BFaces<T> bottom_cell_faces(const T *fw, const T *fs, int n1, int n2, int i, int j,
-                                                       int id) {
-#pragma clang fp contract(fast)
-    BFaces<T> f;
-    f.W = fw[id];
-    f.E = i < n1 - 1 ? fw[id + n2] : T(0);
-    f.S = fs[id];
-    f.N = j < n2 - 1 ? fs[id + 1] : T(0);
-    f.C = -((f.W + f.E) + (f.S + f.N));
-    return f;
-}
-
-// Gauss-Seidel update of cell id = (i, j) from the stored faces and the
-// stored reciprocal rc of the diagonal, in gs_cell's operation order
-template <typename T>
-__device__ __forceinline__ T bottom_gs_f(const T *x, const T *fw, const T *fs, const T *rc, T bv, int n1, int n2,
-                                         int i, int j, int id) {
-#pragma clang fp contract(fast)
-    const BFaces<T> f = bottom_cell_faces(fw, fs, n1, n2, i, j, id);
-    const T xa = i > 0 ? x[id - n2] : T(0), xb = i < n1 - 1 ? x[id + n2] : T(0);
-    const T xS = j > 0 ? x[id - 1] : T(0), xN = j < n2 - 1 ? x[id + 1] : T(0);
-    T s = bv;
-    s -= f.W * xa;
-    s -= f.S * xS;
-    s -= f.E * xb;
-    s -= f.N * xN;
-    return f.C != T(0) ? s * rc[id] : T(0);
-}
-
-// Every level has at most BOTTOM_THREADS cells, so a thread holds at most one
-// cell of each and computes its (i, j) once per level.  The faces of all
-// levels and the reciprocals of their diagonals are formed once, after w is
-// loaded, and read from LDS by every sweep.  Level offsets in LDS are running
-// sums (an array of them indexed by the level would live in scratch memory).
-static_assert(BOTTOM_N * BOTTOM_N <= BOTTOM_THREADS, "one bottom cell per thread and level");
-template <typename T>
-__device__ void mg_bottom_body(const BottomArgs<T> &A) {
-#pragma clang fp contract(fast)
-    __shared__ T sx[BOTTOM_CELLS], sb[BOTTOM_CELLS], sr[BOTTOM_CELLS], sw[BOTTOM_CELLS];
-    __shared__ T sfw[BOTTOM_CELLS], sfs[BOTTOM_CELLS], src[BOTTOM_CELLS];
-    const int t = threadIdx.x;
-    const int nl = A.nl;
-    for (int l = 0, o = 0; l < nl; l++) {
-        const int n1 = A.lev[l].n1, n2 = A.lev[l].n2, ldw = A.lev[l].ldw;
-        const T *w = A.lev[l].w;
-        if (t < n1 * n2) {
-            const int i = t / n2, j = t - i * n2;
-            sw[o + t] = w[(long)i * ldw + j];
-            if (l == 0) sb[t] = A.b[(long)i * A.ldb + j];
-        }
-        o += n1 * n2;
-    }
-    __syncthreads();
-    for (int l = 0, o = 0; l < nl; l++) {
-        const int n1 = A.lev[l].n1, n2 = A.lev[l].n2, hm = A.lev[l].harmonic;
-        const T cx = T(A.lev[l].cx), cy = T(A.lev[l].cy);
-        if (t < n1 * n2) {
-            const int i = t / n2, j = t - i * n2;
-            T W, E, Sf, N;
-            bottom_faces(sw + o, n1, n2, i, j, cx, cy, hm, W, E, Sf, N);
-            const T Cc = -((W + E) + (Sf + N));
-            sfw[o + t] = W;
-            sfs[o + t] = Sf;
-            src[o + t] = Cc != T(0) ? recip(Cc) : T(0);
-        }
-        o += n1 * n2;
-    }
-    __syncthreads();
-    // down: red from zero, black, residual, full weighting
-    int o = 0;   // offset of level l
-    for (int l = 0; l + 1 < nl; l++) {
-        const int n1 = A.lev[l].n1, n2 = A.lev[l].n2, n = n1 * n2;
-        T *x = sx + o, *r = sr + o;
-        const T *b = sb + o, *fw = sfw + o, *fs = sfs + o, *rc = src + o;
-        const bool act = t < n;
-        const int i = t / n2, j = t - i * n2;
-        if (act) {
-            T v = T(0);
-            if (((i + j) & 1) == 0) {
-                const BFaces<T> f = bottom_cell_faces(fw, fs, n1, n2, i, j, t);
-                v = f.C != T(0) ? b[t] * rc[t] : T(0);
-            }
-            x[t] = v;
-        }
-        __syncthreads();
-        if (act && ((i + j) & 1)) x[t] = bottom_gs_f(x, fw, fs, rc, b[t], n1, n2, i, j, t);
-        __syncthreads();
-        for (int pr = 1; pr < A.ns; pr++)   // further red-black pairs
-            for (int c = 0; c <= 1; c++) {
-                if (act && ((i + j) & 1) == c) x[t] = bottom_gs_f(x, fw, fs, rc, b[t], n1, n2, i, j, t);
-                __syncthreads();
-            }
-        if (act) {
-            const BFaces<T> f = bottom_cell_faces(fw, fs, n1, n2, i, j, t);
-            T s = f.C * x[t];
-            s += f.W * (i > 0 ? x[t - n2] : T(0));
-            s += f.S * (j > 0 ? x[t - 1] : T(0));
-            s += f.E * (i < n1 - 1 ? x[t + n2] : T(0));
-            s += f.N * (j < n2 - 1 ? x[t + 1] : T(0));
-            r[t] = b[t] - s;
-        }
-        __syncthreads();
-        const int m1 = A.lev[l + 1].n1, m2 = A.lev[l + 1].n2;
-        T *bc = sb + o + n;
-        if (t < m1 * m2) {
-            const int I = t / m2, J = t - I * m2;
-            const T wL = T((2 * J - 1 >= 0 && 2 * J - 1 < n2) ? pw(2 * J - 1, J, m2) : 0.);
-            const T w0 = T(2 * J < n2 ? pw(2 * J, J, m2) : 0.);
-            const T w1 = T(2 * J + 1 < n2 ? pw(2 * J + 1, J, m2) : 0.);
-            const T wR = T(2 * J + 2 < n2 ? pw(2 * J + 2, J, m2) : 0.);
-            T acc = T(0);
-            for (int f = 2 * I - 1; f <= 2 * I + 2; f++) {
-                if (f < 0 || f >= n1) continue;
-                const T wi = T(pw(f, I, m1));
-                if (wi == T(0)) continue;
-                const T *rf = r + f * n2;
-                const T rL = wL != T(0) ? rf[2 * J - 1] : T(0), r0 = w0 != T(0) ? rf[2 * J] : T(0);
-                const T r1 = w1 != T(0) ? rf[2 * J + 1] : T(0), rR = wR != T(0) ? rf[2 * J + 2] : T(0);
-                const T h = ((wL * rL + w0 * r0) + w1 * r1) + wR * rR;
-                acc += wi * h;
-            }
-            bc[t] = T(0.25) * acc;
-        }
-        __syncthreads();
-        o += n;
-    }
-    // coarsest (o is its offset): k_coarsest's bordered solve (FP64
-    // elimination) of the operator the legs use on that level, assembled from
-    // the faces in LDS
-    if (t == 0) {
-        const int l = nl - 1, n1 = A.lev[l].n1, n2 = A.lev[l].n2, hm = A.lev[l].harmonic;
-        const T cx = T(A.lev[l].cx), cy = T(A.lev[l].cy);
-        const T *b = sb + o, *w = sw + o;
-        T *x = sx + o;
-        // the hierarchy is coarsened until both sides are at most 2
-        if (n1 == 2 && n2 == 2) bottom_coarsest<2, 2>(w, b, x, cx, cy, hm);
-        else if (n1 == 2 && n2 == 1) bottom_coarsest<2, 1>(w, b, x, cx, cy, hm);
-        else if (n1 == 1 && n2 == 2) bottom_coarsest<1, 2>(w, b, x, cx, cy, hm);
-        else if (n1 == 1 && n2 == 1) bottom_coarsest<1, 1>(w, b, x, cx, cy, hm);
-    }
-    __syncthreads();
-    // up: x + P e, black, red
-    for (int l = nl - 2; l >= 0; l--) {
-        const int n1 = A.lev[l].n1, n2 = A.lev[l].n2, n = n1 * n2;
-        const int m1 = A.lev[l + 1].n1, m2 = A.lev[l + 1].n2;
-        const int oc = o;   // offset of level l + 1
-        o -= n;
-        T *x = sx + o;
-        const T *xc = sx + oc, *b = sb + o, *fw = sfw + o, *fs = sfs + o, *rc = src + o;
-        const bool act = t < n;
-        const int i = t / n2, j = t - i * n2;
-        if (act) {
-            int I0 = i >> 1, I1 = (i & 1) ? I0 + 1 : I0 - 1;
-            I0 = I0 > m1 - 1 ? m1 - 1 : I0;
-            I1 = I1 < 0 ? 0 : (I1 > m1 - 1 ? m1 - 1 : I1);
-            const int J = j >> 1;
-            const int Jn = (j & 1) ? (J == m2 - 1 ? J : J + 1) : (J == 0 ? J : J - 1);
-            const T o0 = xc[I0 * m2 + J], o1 = xc[I1 * m2 + J], l0 = xc[I0 * m2 + Jn], l1 = xc[I1 * m2 + Jn];
-            const T e = T(0.5625) * o0 + T(0.1875) * l0 + T(0.1875) * o1 + T(0.0625) * l1;
-            x[t] = x[t] + e;
-        }
-        __syncthreads();
-        for (int pr = 0; pr < A.ns; pr++)
-            for (int c = 1; c >= 0; c--) {
-                if (act && ((i + j) & 1) == c) x[t] = bottom_gs_f(x, fw, fs, rc, b[t], n1, n2, i, j, t);
-                __syncthreads();
-            }
-    }
-    {
-        const int n1 = A.lev[0].n1, n2 = A.lev[0].n2;
-        if (t < n1 * n2) {
-            const int i = t / n2, j = t - i * n2;
-            A.out[(long)i * A.ldo + j] = sx[t];
-        }
-    }
-}
-
-template <typename T>
+// The bottom of the streaming V-cycle (mg_block.h): from the first level of at
+// most 64 x 64 cells down to the coarsest and back up in one workgroup.
+constexpr int BOTTOM_N = 64, BOTTOM_THREADS = 1024;
+template <typename T, bool NINE>
 __global__ void __launch_bounds__(BOTTOM_THREADS) k_mg_bottom(BottomArgs<T> A) {
-    mg_bottom_body<T>(A);
+    __shared__ BotShared<T, NINE> sh;
+    mg_bottom_body<T, NINE>(A, sh);
 }
+static int bottom_threads(int d0) { return d0 == 0 ? BOTTOM_THREADS : 256; }
 
 // first level handled by k_mg_bottom, or -1 when the hierarchy has no level of
 // at most BOTTOM_N x BOTTOM_N cells above its coarsest
 static int bottom_level(const impec_ctx *ctx) {
     if (ctx->P.mg_variant == 2) return -1;
     for (int l = 1; l + 1 < ctx->nlev; l++)
-        if (ctx->lev[l].n1 <= BOTTOM_N && ctx->lev[l].n2 <= BOTTOM_N) {
-            if (ctx->nlev - l > BOTTOM_LEVELS) return -1;
-            int cells = 0;
-            for (int q = l; q < ctx->nlev; q++) cells += ctx->lev[q].n1 * ctx->lev[q].n2;
-            return cells <= BOTTOM_CELLS ? l : -1;
-        }
+        if (ctx->lev[l].n1 <= BOTTOM_N && ctx->lev[l].n2 <= BOTTOM_N) return l;
     return -1;
+}
+// depth (mg_block.h) of a bottom whose first level is L: the levels of depth D
+// have at most 64 >> D cells a side, and the coarsest (at most 2) has depth 5
+static int bottom_depth(const Level &L) {
+    const int s = L.n1 > L.n2 ? L.n1 : L.n2;
+    int d = 0;
+    while (d < 4 && s <= (BOTTOM_N >> (d + 1))) d++;
+    return d;
 }
 
 // levels l < top_level run the streaming legs
@@ -2482,25 +2157,54 @@ static BottomArgs<T> bottom_args(impec_ctx *ctx, int lb) {
     BottomArgs<T> A;
     memset(&A, 0, sizeof(A));
     A.nl = ctx->nlev - lb;
+    A.d0 = bottom_depth(ctx->lev[lb]);
+    A.harmonic = ctx->lev[lb].g.harmonic;
     for (int l = lb; l < ctx->nlev; l++) {
-        const Level &L = ctx->lev[l];
         const FusedArgsT<T> f = fused_args<T>(ctx, l);
-        BottomLev<T> &b = A.lev[l - lb];
+        BotLev<T> &b = A.lev[l - lb];
         b.w = f.w;
         b.ldw = f.ldw;
-        b.n1 = L.n1;
-        b.n2 = L.n2;
-        b.harmonic = L.g.harmonic;
-        b.cx = L.g.cx;
-        b.cy = L.g.cy;
     }
     const Level &B = ctx->lev[lb];
+    A.n1 = B.n1;
+    A.n2 = B.n2;
+    A.cx = B.g.cx;
+    A.cy = B.g.cy;
     A.b = LA::b(B) + B.ld + 1;
     A.ldb = B.ld;
     A.out = LA::r(B) + B.ld + 1;
     A.ldo = B.ld;
     A.ns = mg_ns(ctx);
     A.S = ctx->scal;
+    return A;
+}
+
+// whether level l runs the tile legs of mg_block.h instead of the streaming ones:
+// coarse levels of at most 1024 cells a side.  Step times, ms, of the benchmark's
+// physics without dispersion, streaming legs / tiles to 512 / to 1024 / to 2048:
+// 512^2 1.55 / 1.37 / 1.37 / 1.37, 1024^2 2.13 / 1.87 / 1.86 / 1.87, 2048^2
+// 3.66 / 3.42 / 3.37 / 3.36, 4096^2 9.26 / 9.01 / 8.94 / 9.24.  Above 1024 the
+// launch is bound by bytes again, and the tiles' wider halo costs more.
+#ifndef IMPEC_TILE_MAX
+#define IMPEC_TILE_MAX 1024
+#endif
+constexpr int LEG5_P = 32;
+static bool tile_level(const impec_ctx *ctx, int l) {
+    return l > 0 && ctx->lev[l].n1 <= IMPEC_TILE_MAX && ctx->lev[l].n2 <= IMPEC_TILE_MAX;
+}
+template <typename T>
+static Leg5Args<T> leg5_args(impec_ctx *ctx, int l, int h) {
+    const FusedArgsT<T> f = fused_args<T>(ctx, l);
+    Leg5Args<T> A;
+    memset(&A, 0, sizeof(A));
+    A.w = f.w; A.ldw = f.ldw; A.harmonic = f.g.harmonic;
+    A.cx = f.g.cx; A.cy = f.g.cy;
+    A.n1 = f.g.n1; A.n2 = f.g.n2; A.ld = f.ld;
+    A.b = f.b; A.x = f.x; A.xo = f.xo; A.bc = f.bc; A.xc = f.xc;
+    A.m1 = f.m1; A.m2 = f.m2; A.ldc = f.ldc;
+    A.S = ctx->scal;
+    A.ti = tile_count((A.n1 + 1) / 2, LEG5_P, h);
+    A.tj = tile_count((A.n2 + 1) / 2, LEG5_P, h);
     return A;
 }
 
@@ -2517,7 +2221,10 @@ static int vcycle_fused_ns(impec_ctx *ctx, bool r32, bool skip_first = false) {
     for (int l = skip_first ? 1 : 0; l < ltop; l++) {
         FusedArgsT<T> A = fused_args<T>(ctx, l);
         prof_begin(ctx);
-        if (F && r32 && l == 0 && A.w2 != A.w)
+        if (tile_level(ctx, l)) {
+            const Leg5Args<T> A5 = leg5_args<T>(ctx, l, Halo5<NS>::D);
+            hipLaunchKernelGGL((k_mg5_down<LEG5_P, NS, T>), dim3(A5.ti * A5.tj), dim3(LEG5_P * LEG5_P), 0, ctx->stream, A5);
+        } else if (F && r32 && l == 0 && A.w2 != A.w)
             hipLaunchKernelGGL((k_mg_down<true, true, T, NS, F>), stream_grid(A), blk, 0, ctx->stream, A);
         else if (F && r32 && l == 0)
             hipLaunchKernelGGL((k_mg_down<true, false, T, NS, F>), stream_grid(A), blk, 0, ctx->stream, A);
@@ -2529,7 +2236,8 @@ static int vcycle_fused_ns(impec_ctx *ctx, bool r32, bool skip_first = false) {
     }
     if (lb > 0) {
         prof_begin(ctx);
-        hipLaunchKernelGGL((k_mg_bottom<T>), dim3(1), dim3(BOTTOM_THREADS), 0, ctx->stream, bottom_args<T>(ctx, lb));
+        const BottomArgs<T> B = bottom_args<T>(ctx, lb);
+        hipLaunchKernelGGL((k_mg_bottom<T, false>), dim3(1), dim3(bottom_threads(B.d0)), 0, ctx->stream, B);
         prof_end(ctx, "mg_coarse");
     } else {
         Level &Cl = ctx->lev[L - 1];
@@ -2542,7 +2250,10 @@ static int vcycle_fused_ns(impec_ctx *ctx, bool r32, bool skip_first = false) {
     for (int l = ltop - 1; l >= 0; l--) {
         FusedArgsT<T> A = fused_args<T>(ctx, l);
         prof_begin(ctx);
-        if (F && r32 && l == 0 && A.w2 != A.w)
+        if (tile_level(ctx, l)) {
+            const Leg5Args<T> A5 = leg5_args<T>(ctx, l, Halo5<NS>::U);
+            hipLaunchKernelGGL((k_mg5_up<LEG5_P, NS, T>), dim3(A5.ti * A5.tj), dim3(LEG5_P * LEG5_P), 0, ctx->stream, A5);
+        } else if (F && r32 && l == 0 && A.w2 != A.w)
             hipLaunchKernelGGL((k_mg_up<true, true, T, NS, F>), stream_grid(A), blk, 0, ctx->stream, A);
         else if (F && r32 && l == 0)
             hipLaunchKernelGGL((k_mg_up<true, false, T, NS, F>), stream_grid(A), blk, 0, ctx->stream, A);
@@ -2585,7 +2296,7 @@ constexpr int LEG9_P = 32;   // blocks a side of a tile
 
 static OpPlanes<double> op_planes(const Level &L) { return OpPlanes<double>{L.a9, L.plane9, L.ld9}; }
 
-// first level handled by k_mg9_bottom
+// first level handled by k_mg_bottom
 static int bottom_level9(const impec_ctx *ctx) {
     int l = 1;
     while (ctx->lev[l].n1 > 64 || ctx->lev[l].n2 > 64) l++;
@@ -2658,19 +2369,16 @@ static Leg9Args leg9_args(const impec_ctx *ctx, int l, int hi, int hj) {
     return A;
 }
 
-static Bot9Args bot9_args(const impec_ctx *ctx, int lb) {
-    Bot9Args A;
+static BottomArgs<double> bottom_args9(const impec_ctx *ctx, int lb) {
+    BottomArgs<double> A;
     memset(&A, 0, sizeof(A));
     const Level &B = ctx->lev[lb];
-    const int s = B.n1 > B.n2 ? B.n1 : B.n2;
-    A.d0 = 0;
-    while (A.d0 < 4 && s <= (64 >> (A.d0 + 1))) A.d0++;
+    A.d0 = bottom_depth(B);
     A.nl = ctx->nlev - lb;
-    for (int l = lb; l < ctx->nlev; l++) {
-        A.lev[l - lb].A = op_planes(ctx->lev[l]);
-        A.lev[l - lb].n1 = ctx->lev[l].n1;
-        A.lev[l - lb].n2 = ctx->lev[l].n2;
-    }
+    A.ns = mg_ns(ctx);
+    for (int l = lb; l < ctx->nlev; l++) A.lev[l - lb].A = op_planes(ctx->lev[l]);
+    A.n1 = B.n1;
+    A.n2 = B.n2;
     A.inv = ctx->op9_inv;
     A.b = B.b + B.ld + 1;
     A.out = B.r + B.ld + 1;
@@ -2693,9 +2401,9 @@ static int vcycle9(impec_ctx *ctx, int *parts) {
         else hipLaunchKernelGGL((k_mg9_down<LEG9_P, NS, false>), dim3(A.ti * A.tj), blk, 0, ctx->stream, A);
         prof_end(ctx, l == 0 ? "mg_down_l0" : "mg_coarse");
     }
-    const Bot9Args B = bot9_args(ctx, lb);
+    const BottomArgs<double> B = bottom_args9(ctx, lb);
     prof_begin(ctx);
-    hipLaunchKernelGGL((k_mg9_bottom<NS>), dim3(1), dim3(B.d0 == 0 ? 1024 : 256), 0, ctx->stream, B);
+    hipLaunchKernelGGL((k_mg_bottom<double, true>), dim3(1), dim3(bottom_threads(B.d0)), 0, ctx->stream, B);
     prof_end(ctx, "mg_coarse");
     for (int l = lb - 1; l >= 0; l--) {
         const Leg9Args A = leg9_args(ctx, l, H::UI, H::UJ);
@@ -3395,7 +3103,8 @@ struct ShiftRec {
 
 template <typename T>
 struct LegTabs {
-    Batch<FusedArgsT<T>> down[MAX_LEVELS], up[MAX_LEVELS];
+    Batch<FusedArgsT<T>> down[MAX_LEVELS], up[MAX_LEVELS];   // streaming legs
+    Batch<Leg5Args<T>> tdown[MAX_LEVELS], tup[MAX_LEVELS];   // tile legs
     Batch<CoarsestRec<T>> coarsest;    // members without a bottom kernel
     Batch<BottomArgs<T>> bottom;       // members with one
     Batch<DirMvArgs<T>> dir;
@@ -3403,6 +3112,8 @@ struct LegTabs {
         for (int l = 0; l < MAX_LEVELS; l++) {
             batch_free(down[l]);
             batch_free(up[l]);
+            batch_free(tdown[l]);
+            batch_free(tup[l]);
         }
         batch_free(coarsest);
         batch_free(bottom);
@@ -3495,11 +3206,31 @@ __global__ void __launch_bounds__(64 * SW_WAVES)
     if (!in_state(A.S, need)) return;
     mg_up_body<FINE0, false, T, NS>(A, gw - start[m]);
 }
+// tile legs of one level over every member in state `need`, one workgroup per tile
+template <typename T, int NS>
+__global__ void __launch_bounds__(LEG5_P *LEG5_P) kb_mg5_down(const Leg5Args<T> *__restrict__ tab,
+                                                             const int *__restrict__ start, int nmem, int need) {
+    __shared__ T sm[BlkGeo<LEG5_P>::CELLS];
+    const int m = member_of(start, nmem, blockIdx.x);
+    const Leg5Args<T> &A = tab[m];
+    if (!in_state(A.S, need)) return;
+    leg5_down_body<LEG5_P, NS, T>(A, blockIdx.x - start[m], sm);
+}
+template <typename T, int NS>
+__global__ void __launch_bounds__(LEG5_P *LEG5_P) kb_mg5_up(const Leg5Args<T> *__restrict__ tab,
+                                                           const int *__restrict__ start, int nmem, int need) {
+    __shared__ T sm[BlkGeo<LEG5_P>::CELLS];
+    const int m = member_of(start, nmem, blockIdx.x);
+    const Leg5Args<T> &A = tab[m];
+    if (!in_state(A.S, need)) return;
+    leg5_up_body<LEG5_P, NS, T>(A, blockIdx.x - start[m], sm);
+}
 template <typename T>
 __global__ void __launch_bounds__(BOTTOM_THREADS) kb_mg_bottom(const BottomArgs<T> *__restrict__ tab, int need) {
     const BottomArgs<T> &A = tab[blockIdx.x];
     if (!in_state(A.S, need)) return;
-    mg_bottom_body<T>(A);
+    __shared__ BotShared<T, false> sh;
+    mg_bottom_body<T, false>(A, sh);
 }
 template <typename T>
 __global__ void kb_coarsest(const CoarsestRec<T> *__restrict__ tab, int need) {
@@ -3760,15 +3491,26 @@ static int build_legs(impec_ensemble *e, LegTabs<T> &t) {
     const int lmax = e->pres->lmax;
     for (int l = 0; l + 1 < lmax; l++) {
         std::vector<FusedArgsT<T>> recs(n);
-        std::vector<int> units(n, 0);
+        std::vector<Leg5Args<T>> td(n), tu(n);
+        std::vector<int> units(n, 0), ud(n, 0), uu(n, 0);
         for (int k = 0; k < n; k++) {
             impec_ctx *ctx = e->m[k];
             if (l >= top_level(ctx)) continue;
+            if (tile_level(ctx, l)) {   // as the members' own cycles
+                const bool two = mg_ns(ctx) == 2;
+                td[k] = leg5_args<T>(ctx, l, two ? Halo5<2>::D : Halo5<1>::D);
+                tu[k] = leg5_args<T>(ctx, l, two ? Halo5<2>::U : Halo5<1>::U);
+                ud[k] = td[k].ti * td[k].tj;
+                uu[k] = tu[k].ti * tu[k].tj;
+                continue;
+            }
             recs[k] = fused_args<T>(ctx, l);
             units[k] = recs[k].nwave;
         }
         ENS_CHECK(e, batch_upload(t.down[l], recs, units));
         ENS_CHECK(e, batch_upload(t.up[l], recs, units));
+        ENS_CHECK(e, batch_upload(t.tdown[l], td, ud));
+        ENS_CHECK(e, batch_upload(t.tup[l], tu, uu));
     }
     std::vector<CoarsestRec<T>> cr(n);
     std::vector<BottomArgs<T>> br(n);
@@ -3838,7 +3580,7 @@ static int build_lists(impec_ensemble *e) {
     if ((st = make_list(e, dstart, all, t->h_iter[t->lmax]))) return st;
     for (int l = 0; l + 1 < t->lmax; l++) {
         std::vector<int> u(n, 0);
-        for (int k = 0; k < n; k++) u[k] = l < top_level(e->m[k]);
+        for (int k = 0; k < n; k++) u[k] = l < top_level(e->m[k]) && !tile_level(e->m[k], l);
         const int *ls = t->mixed ? t->l32.down[l].start : t->l64.down[l].start;
         if ((st = make_list(e, ls, u, t->h_iter[1 + l]))) return st;
     }
@@ -3993,6 +3735,16 @@ static hipError_t launch_t(void (*k)(const E *, int), const Batch<E> &b, hipStre
     return hipGetLastError();
 }
 
+// the tile legs of level l of the members in state `need`
+template <typename T, int NS>
+static void ens_tile_leg(impec_ensemble *e, const LegTabs<T> &t, int l, bool up, int need) {
+    const Batch<Leg5Args<T>> &b = up ? t.tup[l] : t.tdown[l];
+    if (b.nmem == 0) return;
+    const dim3 blk(LEG5_P * LEG5_P);
+    if (up) hipLaunchKernelGGL((kb_mg5_up<T, NS>), dim3(b.total), blk, 0, e->stream, b.tab, b.start, b.nmem, need);
+    else hipLaunchKernelGGL((kb_mg5_down<T, NS>), dim3(b.total), blk, 0, e->stream, b.tab, b.start, b.nmem, need);
+}
+
 // the legs of one V-cycle of every member in state `need` (-1: all); the
 // members share the number of red-black pairs per leg
 template <typename T, int NS>
@@ -4002,6 +3754,7 @@ static int ens_vcycle_ns(impec_ensemble *e, const LegTabs<T> &t, int need) {
     hipStream_t s = e->stream;
     for (int l = 0; l + 1 < lmax; l++) {
         const Batch<FusedArgsT<T>> &b = t.down[l];
+        ens_tile_leg<T, NS>(e, t, l, false, need);
         if (b.nmem == 0) continue;
         const dim3 g((b.total + SW_WAVES - 1) / SW_WAVES);
         if (l == 0) hipLaunchKernelGGL((kb_mg_down<true, T, NS>), g, blk, 0, s, b.tab, b.start, b.nmem, b.total, need);
@@ -4011,6 +3764,7 @@ static int ens_vcycle_ns(impec_ensemble *e, const LegTabs<T> &t, int need) {
     ENS_CHECK(e, launch_m(kb_mg_bottom<T>, t.bottom, dim3(BOTTOM_THREADS), s, need));
     for (int l = lmax - 2; l >= 0; l--) {
         const Batch<FusedArgsT<T>> &b = t.up[l];
+        ens_tile_leg<T, NS>(e, t, l, true, need);
         if (b.nmem == 0) continue;
         const dim3 g((b.total + SW_WAVES - 1) / SW_WAVES);
         if (l == 0) hipLaunchKernelGGL((kb_mg_up<true, T, NS>), g, blk, 0, s, b.tab, b.start, b.nmem, b.total, need);
@@ -4053,6 +3807,8 @@ static int ens_cg_slot_t(impec_ensemble *e, const LegTabs<T> &lt) {
     const int ns = mg_ns(e->m[0]);
     for (int l = 0; l + 1 < lmax; l++) {
         const Batch<FusedArgsT<T>> &b = lt.down[l];
+        if (ns == 2) ens_tile_leg<T, 2>(e, lt, l, false, (int)EST_ITER);
+        else ens_tile_leg<T, 1>(e, lt, l, false, (int)EST_ITER);
         if (b.nmem == 0) continue;
         const dim3 g(persist_grid((b.total + SW_WAVES - 1) / SW_WAVES, PERSIST_LEG_WG));
         const ActList &a = t->h_iter[1 + l].act;
@@ -4068,6 +3824,8 @@ static int ens_cg_slot_t(impec_ensemble *e, const LegTabs<T> &lt) {
     ENS_CHECK(e, launch_m(kb_mg_bottom<T>, lt.bottom, dim3(BOTTOM_THREADS), s, (int)EST_ITER));
     for (int l = lmax - 2; l >= 0; l--) {
         const Batch<FusedArgsT<T>> &b = lt.up[l];
+        if (ns == 2) ens_tile_leg<T, 2>(e, lt, l, true, (int)EST_ITER);
+        else ens_tile_leg<T, 1>(e, lt, l, true, (int)EST_ITER);
         if (b.nmem == 0) continue;
         const dim3 g(persist_grid((b.total + SW_WAVES - 1) / SW_WAVES, PERSIST_LEG_WG));
         const ActList &a = t->h_iter[1 + l].act;
