@@ -206,7 +206,10 @@ int impec::ctx_create(const impec_params *P, hipStream_t ext, impec_ctx **out) {
     if (ext) ctx->stream = ext;
     else if (hipStreamCreate(&ctx->stream) != hipSuccess) st = set_error(ctx, IMPEC_EHIP, "stream");
     else ctx->own_stream = 1;
-    if (!st && (hipEventCreate(&ctx->ev0) != hipSuccess || hipEventCreate(&ctx->ev1) != hipSuccess))
+    transfer_attach();
+    if (!st && (hipEventCreate(&ctx->ev0) != hipSuccess || hipEventCreate(&ctx->ev1) != hipSuccess ||
+                hipEventCreateWithFlags(&ctx->ev_get[0], hipEventDisableTiming) != hipSuccess ||
+                hipEventCreateWithFlags(&ctx->ev_get[1], hipEventDisableTiming) != hipSuccess))
         st = set_error(ctx, IMPEC_EHIP, "events");
     const size_t ns = scalar_elems(ctx), nv = vel_elems(ctx), nq = (size_t)ctx->N1 * ctx->N2;
     if (!st) st = dalloc(ctx, &ctx->c, ns);
@@ -265,6 +268,9 @@ int impec_destroy(impec_ctx *ctx) {
     if (ctx->h_scal) hipHostFree(ctx->h_scal);
     if (ctx->ev0) hipEventDestroy(ctx->ev0);
     if (ctx->ev1) hipEventDestroy(ctx->ev1);
+    for (hipEvent_t ev : ctx->ev_get)
+        if (ev) hipEventDestroy(ev);
+    transfer_detach();
     if (ctx->stream && ctx->own_stream) hipStreamDestroy(ctx->stream);
     free(ctx);
     return IMPEC_OK;
@@ -283,20 +289,13 @@ static int put2d(impec_ctx *ctx, double *dst, int ld_dst, const double *src, int
     IMPEC_HIP_CHECK(ctx, hipStreamSynchronize(ctx->stream));
     return IMPEC_OK;
 }
-static int get2d(impec_ctx *ctx, double *dst, const double *src, int ld_src, int rows, int cols) {
-    IMPEC_HIP_CHECK(ctx, hipMemcpy2DAsync(dst, sizeof(double) * cols, src, sizeof(double) * ld_src, sizeof(double) * cols,
-                                          rows, hipMemcpyDeviceToHost, ctx->stream));
-    IMPEC_HIP_CHECK(ctx, hipStreamSynchronize(ctx->stream));
-    return IMPEC_OK;
-}
-
 int impec_set_concentration(impec_ctx *ctx, const double *c) {
     if (!ctx || !c) return IMPEC_EINVAL;
     return put2d(ctx, ctx->c, ctx->lds, c, ctx->N1 + 2 * ctx->B, ctx->N2 + 2 * ctx->B);
 }
 int impec_get_concentration(impec_ctx *ctx, double *c) {
     if (!ctx || !c) return IMPEC_EINVAL;
-    return get2d(ctx, c, ctx->c, ctx->lds, ctx->N1 + 2 * ctx->B, ctx->N2 + 2 * ctx->B);
+    return get_field(ctx, c, ctx->c, nullptr, ctx->lds, ctx->N1 + 2 * ctx->B, ctx->N2 + 2 * ctx->B);
 }
 int impec_set_pressure(impec_ctx *ctx, const double *p) {
     if (!ctx || !p) return IMPEC_EINVAL;
@@ -306,7 +305,7 @@ int impec_set_pressure(impec_ctx *ctx, const double *p) {
 }
 int impec_get_pressure(impec_ctx *ctx, double *p) {
     if (!ctx || !p) return IMPEC_EINVAL;
-    return get2d(ctx, p, ctx->p, ctx->lds, ctx->N1 + 2 * ctx->B, ctx->N2 + 2 * ctx->B);
+    return get_field(ctx, p, ctx->p, nullptr, ctx->lds, ctx->N1 + 2 * ctx->B, ctx->N2 + 2 * ctx->B);
 }
 
 // interleaved host velocity <-> two device component arrays
@@ -324,16 +323,7 @@ int impec_set_velocity(impec_ctx *ctx, const double *v) {
 }
 int impec_get_velocity(impec_ctx *ctx, double *v) {
     if (!ctx || !v) return IMPEC_EINVAL;
-    const int rows = ctx->N1 + 1 + 2 * ctx->B, cols = ctx->N2 + 1 + 2 * ctx->B;
-    std::vector<double> a((size_t)rows * cols), b((size_t)rows * cols);
-    int st = get2d(ctx, a.data(), ctx->u, ctx->ldv, rows, cols);
-    if (!st) st = get2d(ctx, b.data(), ctx->v, ctx->ldv, rows, cols);
-    if (st) return st;
-    for (size_t k = 0; k < a.size(); k++) {
-        v[2 * k] = a[k];
-        v[2 * k + 1] = b[k];
-    }
-    return IMPEC_OK;
+    return get_field(ctx, v, ctx->u, ctx->v, ctx->ldv, ctx->N1 + 1 + 2 * ctx->B, ctx->N2 + 1 + 2 * ctx->B);
 }
 
 int impec_set_source(impec_ctx *ctx, const double *q) {

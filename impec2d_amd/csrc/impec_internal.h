@@ -209,6 +209,7 @@ struct impec_ctx {
     impec::ProfEntry prof[32];
     int nprof;
     hipEvent_t ev0, ev1;
+    hipEvent_t ev_get[2];      // the two staging halves of get_field
     int own_stream;            // 0 when the stream belongs to an ensemble
 };
 
@@ -285,6 +286,14 @@ inline long chunk_rows(long n, long nstrip, long target, bool capped) {
 inline size_t sidx(const impec_ctx *ctx, int i, int j) {
     return (size_t)(i + ctx->B) * ctx->lds + (j + ctx->B);
 }
+
+// ---- fields to the host (transfer.hip) ----
+// the host layout (rows x cols, compact) of device array a with pitch ld, or of
+// a and b interleaved (b not null); waits for the stream
+int get_field(impec_ctx *ctx, double *dst, const double *a, const double *b, int ld, int rows, int cols);
+// the number of contexts that may call it: the last one to go frees the staging memory
+void transfer_attach();
+void transfer_detach();
 
 // ---- field kernels (k_field.hip) ----
 int launch_fill_scalar(impec_ctx *ctx, double *a, int periodic);
