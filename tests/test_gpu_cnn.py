@@ -99,3 +99,25 @@ def test_learned_guess_trains_and_keeps_tolerance(gpu_lib):
          "learned", res[capi.GUESS_LEARNED])
     assert sum(res[capi.GUESS_EXTRAPOLATE]) <= sum(res[capi.GUESS_PREVIOUS]) + 2
     assert sum(res[capi.GUESS_LEARNED]) <= sum(res[capi.GUESS_EXTRAPOLATE]) + steps
+
+
+@pytest.mark.parametrize("n,h,w", [(1, 3, 31), (1, 4, 32), (1, 5, 33), (2, 9, 70), (40, 64, 64)])
+def test_weight_gradients_over_tiles(gpu_lib, n, h, w):
+    """The 32 -> 32 layer's weight gradient over less than one 4 x 32 tile, ragged
+    tiles and more tiles than workgroups.  Three layers: its inputs differ from
+    the oracle's only where FP32 and FP64 round a BF16 value differently (about
+    one value in 10^4, by 2^-8: 3e-5 of the norm) and by the order of the FP32
+    sums (below 1e-5), hence 1e-3; a lost or doubled tile is at least
+    (1280 tiles)^-1/2 = 3e-2."""
+    from impec2d_amd import capi
+    net = capi.Network(layers=3, capacity=4, crop=32, seed=5)
+    rng = np.random.default_rng(n * 100 + w)
+    p = co.bf16((rng.standard_normal(net.nparam) * 0.2).astype(np.float32))
+    net.set_params(p)
+    x = rng.standard_normal((n, h, w, 3)).astype(np.float32)
+    t = rng.standard_normal((n, h, w)).astype(np.float32)
+    g, _ = net.gradients(x, t)
+    go, _ = co.gradients(p.astype(np.float64), x, t, 3, bf16_mode=True, kind="h1")
+    _, offs, _ = co.layout(3)
+    for wo, end in ((offs[1][0], offs[1][1]), (offs[1][1], offs[2][0])):
+        assert _rel(g[wo:end], go[wo:end]) < 1e-3, _rel(g[wo:end], go[wo:end])
