@@ -529,11 +529,17 @@ int launch_cfl(impec_ctx *ctx, double *dt_out) {
 // sum runs over the sinks in row-major order on one thread when there are few
 // of them (the reference's order), as a block tree otherwise.
 // ---------------------------------------------------------------------------
+constexpr int TR_ORDERED = 4096;
 template <class G>
 __device__ __forceinline__ void tr_body(const G &gr_, double *__restrict__ c, const int *__restrict__ idx, const double *__restrict__ qv, int nsrc,
                      int N2, int B, int ld, double dt, double hdt, double inj, double *__restrict__ scal,
                      double *__restrict__ md) {
     const int t = threadIdx.x;
+    // the ordered sum of up to TR_ORDERED terms runs over LDS (a global load
+    // per term, one after the other, took 250 us for the 2540 well cells of the
+    // 566^2 grid; 11 us so, the additions' own latency)
+    __shared__ __attribute__((aligned(16))) double smd[TR_ORDERED];
+    const bool ordered = nsrc <= TR_ORDERED;
     for (int k = t; k < nsrc; k += blockDim.x) {
         const int cell = idx[k];
         const int i = cell / N2, j = cell - i * N2;
@@ -547,14 +553,23 @@ __device__ __forceinline__ void tr_body(const G &gr_, double *__restrict__ c, co
         } else if (qij > 0) {
             *cij += dt * inj * qij;
         }
-        md[k] = d;
+        if (ordered) smd[k] = d;
+        else md[k] = d;
     }
     __syncthreads();
     double tmo[1] = {0.};
-    if (nsrc <= 4096) {
-        if (t == 0)
-            for (int k = 0; k < nsrc; k++)
-                if (qv[k] < 0) tmo[0] += md[k];
+    if (ordered) {
+        if (t == 0) {   // an injector's term is zero and leaves the sum unchanged
+            int k = 0;
+            for (; k + 8 <= nsrc; k += 8) {
+                double v[8];
+#pragma unroll
+                for (int u = 0; u < 8; u++) v[u] = smd[k + u];
+#pragma unroll
+                for (int u = 0; u < 8; u++) tmo[0] += v[u];
+            }
+            for (; k < nsrc; k++) tmo[0] += smd[k];
+        }
         __syncthreads();
     } else {
         for (int k = t; k < nsrc; k += blockDim.x) tmo[0] += md[k];
