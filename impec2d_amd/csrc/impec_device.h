@@ -145,6 +145,51 @@ __device__ __forceinline__ void strided_combine_nv(const double *__restrict__ p,
     }
 }
 
+// Sums of NV vectors p + q * vstride of n <= FOLD_MAX partials by a workgroup of
+// 256 threads, every thread getting all NV: for kernels that need the sums of the
+// launch before them and are few enough workgroups to form them each for itself,
+// in place of a launch of one workgroup between the two.  The result is that
+// launch's bit for bit (strided_combine over 1024 threads, then block_reduce):
+// thread t stands for its threads t, t + 256, t + 512 and t + 768.
+constexpr int FOLD_MAX = 4096;
+template <int NV>
+__device__ __forceinline__ void fold_sums(const double *__restrict__ p, long vstride, int n, double (&out)[NV]) {
+    __shared__ double sh[NV][16];
+    const int t = tid_linear(), lane = t & (WAVE - 1), wv = t / WAVE;
+    double v[NV][4];
+#pragma unroll
+    for (int q = 0; q < NV; q++)
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            double a = 0.;
+#pragma unroll
+            for (int u = 0; u < FOLD_MAX / 1024; u++) {
+                const int b = t + 256 * k + 1024 * u;
+                a += b < n ? p[q * vstride + b] : 0.;
+            }
+            v[q][k] = a;
+        }
+#pragma unroll
+    for (int off = WAVE / 2; off > 0; off >>= 1)
+#pragma unroll
+        for (int q = 0; q < NV; q++)
+#pragma unroll
+            for (int k = 0; k < 4; k++) v[q][k] += __shfl_down(v[q][k], off, WAVE);
+    if (lane == 0)
+#pragma unroll
+        for (int q = 0; q < NV; q++)
+#pragma unroll
+            for (int k = 0; k < 4; k++) sh[q][4 * k + wv] = v[q][k];
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < NV; q++) {
+        double s = sh[q][0];
+#pragma unroll
+        for (int w = 1; w < 16; w++) s += sh[q][w];
+        out[q] = s;
+    }
+}
+
 // mu(c) of EllipticSolver.cpp:692-695
 __device__ __forceinline__ double mu_of(double c, double mob1over4, double mu_res) {
     double x = (1. - c + mob1over4 * c);

@@ -28,7 +28,9 @@ enum Scal {
     S_RHO = 0, S_RHO_OLD = 1, S_DQ = 2, S_RR = 3, S_RSUM = 4, S_ZSUM = 5, S_ALPHA = 6, S_BETA = 7,
     S_OMEGA = 8, S_TS = 9, S_TT = 10,
     S_FLOOR = 11,     // with S_TT: || |b| + |A| |p| ||^2, the rounding scale of the true residual
-    S_XPIN = 12, S_RX = 14, S_BB = 15, S_R0V = 19,
+    S_XPIN = 12,
+    S_RHO_NEXT = 13,  // r.z of the iteration under way, until its update makes it S_RHO
+    S_RX = 14, S_BB = 15, S_R0V = 19,
     S_MASS = 16, S_DIV = 17, S_NOFLOW = 18,          // written together by the diagnostics pass
     S_MAXVEL = 20, S_MINDT = 21, S_MINDT_DIFF = 22,  // CFL pass
     S_OUTFLUX = 24, S_TMO = 25, S_CMAX = 26, S_CMIN = 27,
@@ -349,7 +351,8 @@ int cn_operator_dump(impec_ctx *ctx, double dt, double *A9_host, double *rhs_hos
 
 // ---- reductions (k_field.hip) ----
 // sum of NV per-block partial vectors into scal[dst .. dst+NV)
-int finish_sum(impec_ctx *ctx, int nblocks, int nv, int dst, PubArgs pub = PubArgs{nullptr, 0});
+// (vec: the first of them in the part buffer)
+int finish_sum(impec_ctx *ctx, int nblocks, int nv, int dst, PubArgs pub = PubArgs{nullptr, 0}, int vec = 0);
 
 // ---- ensembles: batched launches (k_field.hip, k_pressure.hip, k_transport.hip) ----
 int ens_set_error(impec_ensemble *e, int code, const char *fmt, ...);

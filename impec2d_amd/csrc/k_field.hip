@@ -333,6 +333,17 @@ int launch_velocity(impec_ctx *ctx) {
 template <int OP, class G>
 __device__ __forceinline__ void finish_body(const G &gr_, const double *__restrict__ part, int nblocks, int nv, double *__restrict__ scal,
                          int dst) {
+    if (nv == 2) {   // both at once, in the same order
+        double v[2];
+        strided_combine_nv<OP, 2>(part, RED_BLOCKS, nblocks, v);
+        block_reduce<OP, 2>(v);
+        if (threadIdx.x == 0) {
+            scal[dst] = v[0];
+            scal[dst + 1] = v[1];
+        }
+        __syncthreads();
+        return;
+    }
     for (int k = 0; k < nv; k++) {
         double v[1] = {strided_combine<OP>(part + k * RED_BLOCKS, nblocks)};
         block_reduce<OP, 1>(v);
@@ -374,22 +385,23 @@ __global__ void __launch_bounds__(FIN_THREADS) k_finish_reduce(const double *__r
 }
 
 template <int OP>
-static int finish_op(impec_ctx *ctx, int nblocks, int nv, int dst, PubArgs pub = PubArgs{nullptr, 0}) {
+static int finish_op(impec_ctx *ctx, int nblocks, int nv, int dst, PubArgs pub = PubArgs{nullptr, 0}, int vec = 0) {
+    const double *part = ctx->part + (size_t)vec * RED_BLOCKS;
     if (nblocks > 8 * FIN_THREADS && nv <= PART_VECS) {
         hipLaunchKernelGGL(k_finish_shares<OP>, dim3(FIN_THREADS / FIN_STAGE_WG), dim3(FIN_STAGE_WG), 0, ctx->stream,
-                           ctx->part, nblocks, nv, ctx->part_mid);
+                           part, nblocks, nv, ctx->part_mid);
         hipLaunchKernelGGL(k_finish_reduce<OP>, dim3(1), dim3(FIN_THREADS), 0, ctx->stream, ctx->part_mid, nv,
                            ctx->scal, dst, pub);
     } else {
-        hipLaunchKernelGGL(k_finish<OP>, dim3(1), dim3(FIN_THREADS), 0, ctx->stream, ctx->part, nblocks, nv, ctx->scal,
+        hipLaunchKernelGGL(k_finish<OP>, dim3(1), dim3(FIN_THREADS), 0, ctx->stream, part, nblocks, nv, ctx->scal,
                            dst, pub);
     }
     IMPEC_HIP_CHECK(ctx, hipGetLastError());
     return IMPEC_OK;
 }
 
-int finish_sum(impec_ctx *ctx, int nblocks, int nv, int dst, PubArgs pub) {
-    return finish_op<RED_SUM>(ctx, nblocks, nv, dst, pub);
+int finish_sum(impec_ctx *ctx, int nblocks, int nv, int dst, PubArgs pub, int vec) {
+    return finish_op<RED_SUM>(ctx, nblocks, nv, dst, pub, vec);
 }
 
 static int red_blocks(long long n) {

@@ -1660,6 +1660,59 @@ constexpr int DM_OUT = 62, DM_PF = IMPEC_DM_PF;
 #define IMPEC_DM_WAVES_F32 6144
 #endif
 
+// The sums a CG kernel needs of the launch before it.  n > 0: their n partials
+// (fold_sums forms them in every workgroup; the first one keeps them in S);
+// n = 0: they are in S already (k_finish_rho, finish_sum).  The partials of the
+// V-cycle, the matvec and the update are different vectors of the part buffer:
+// a kernel's workgroups write theirs while others still read the previous ones.
+struct Fold {
+    const double *part;
+    int n;
+    double *S;
+    double inv_n;
+};
+constexpr int PART_CYCLE = 0, PART_DQ = 2, PART_RR = 3;
+static_assert(PART_RR + 2 <= PART_VECS, "vectors of the CG's partial sums");
+
+// mean of the V-cycle's output and beta of the direction update
+template <bool FOLD>
+__device__ __forceinline__ void dir_scalars(const CgArgs &c, const Fold &f, const double *__restrict__ S, int first,
+                                            double &mean, double &beta) {
+    if constexpr (FOLD) {
+        double v[2];
+        fold_sums<2>(f.part, RED_BLOCKS, f.n, v);
+        const double rho = v[1] - v[0] * f.inv_n * S[S_RSUM];
+        mean = v[0] / (double)c.n;
+        beta = first ? 0. : rho / S[S_RHO];   // S_RHO: the previous iteration's until this one's update
+        if (tid_linear() == 0 && blockIdx.x == 0 && blockIdx.y == 0) {
+            f.S[S_ZSUM] = v[0];
+            f.S[S_RX] = v[1];
+            f.S[S_RHO_NEXT] = rho;
+        }
+    } else {
+        mean = S[S_ZSUM] / (double)c.n;
+        beta = first ? 0. : S[S_RHO] / S[S_RHO_OLD];
+    }
+}
+
+// alpha of the update (cg_alpha)
+template <bool FOLD>
+__device__ __forceinline__ double update_alpha(const Fold &f, const double *__restrict__ S) {
+    if constexpr (FOLD) {
+        double v[1];
+        fold_sums<1>(f.part, RED_BLOCKS, f.n, v);
+        const double dq = v[0], rho = S[S_RHO_NEXT], a = rho / dq;
+        if (tid_linear() == 0 && blockIdx.x == 0 && blockIdx.y == 0) {
+            f.S[S_RHO_OLD] = f.S[S_RHO];
+            f.S[S_RHO] = rho;
+            f.S[S_DQ] = dq;
+        }
+        return (fabs(dq) > 0. && isfinite(a)) ? a : 0.;
+    } else {
+        return cg_alpha(S);
+    }
+}
+
 // DT: storage of d and q, double for the FP64 CG, float for the FP32-vector CG
 // (whose matvec reads FP32 copies of the face mobilities, fx32 / fy32)
 template <typename T, typename DT = double>
@@ -1690,7 +1743,8 @@ __device__ __forceinline__ void op_row5_f32(const LevArgs &L, const float *fx, c
 
 template <typename T, typename DT = double>
 __device__ __forceinline__ void dir_mv_body(const DirMvArgs<T, DT> &A, const DT *__restrict__ dold,
-                                            DT *__restrict__ dnew, const int first, const int wid) {
+                                            DT *__restrict__ dnew, const int first, const int wid, const double mean,
+                                            const double beta) {
     if (wid >= A.nwave) return;
     const CgArgs &c = A.c;
     const int n1 = c.n1, n2 = c.n2;
@@ -1701,8 +1755,6 @@ __device__ __forceinline__ void dir_mv_body(const DirMvArgs<T, DT> &A, const DT 
     const int jc = j < 0 ? 0 : (j > n2 - 1 ? n2 - 1 : j);
     const bool outl = lane >= 1 && lane <= DM_OUT && jv;
     const int i0 = chunk * A.R, i1 = i0 + A.R < n1 ? i0 + A.R : n1;
-    const double mean = A.S[S_ZSUM] / (double)c.n;
-    const double beta = first ? 0. : A.S[S_RHO] / A.S[S_RHO_OLD];
     const long ld = c.ld;
     const T *__restrict__ x0 = A.x0;
     auto row_of = [&](int i) -> long { const int ic = i < 0 ? 0 : (i > n1 - 1 ? n1 - 1 : i); return (long)(ic + 1) * ld + (jc + 1); };
@@ -1765,22 +1817,26 @@ __device__ __forceinline__ void dir_mv_body(const DirMvArgs<T, DT> &A, const DT 
     if (lane == 0) A.part[wid] = acc;
 }
 
-template <typename T, typename DT = double>
+template <typename T, typename DT, bool FOLD>
 __global__ void __launch_bounds__(64 * SW_WAVES) k_dir_mv(DirMvArgs<T, DT> A, const DT *__restrict__ dold,
-                                                          DT *__restrict__ dnew, int first) {
-    dir_mv_body<T, DT>(A, dold, dnew, first, xcd_wave());
+                                                          DT *__restrict__ dnew, int first, Fold f) {
+    static_assert(!FOLD || SW_WAVES == 4, "fold_sums runs on 256 threads");
+    double mean, beta;
+    dir_scalars<FOLD>(A.c, f, A.S, first, mean, beta);
+    dir_mv_body<T, DT>(A, dold, dnew, first, xcd_wave(), mean, beta);
 }
 
 // The direction update and matvec of k_dir_mv for the assembled 9-point
 // operator, one cell per thread: d_new at the cell's nine points is formed from
 // the V-cycle output and the old direction (cached: every value is read by nine
 // threads), and the cell's own is stored.
+template <bool FOLD>
 __global__ void __launch_bounds__(256) k_dir_mv9(OpPlanes<double> A, CgArgs c, const double *__restrict__ x0,
                                                  const double *__restrict__ dold, double *__restrict__ dnew,
                                                  double *__restrict__ qv, const double *__restrict__ S, int first,
-                                                 double *__restrict__ part) {
-    const double mean = S[S_ZSUM] / (double)c.n;
-    const double beta = first ? 0. : S[S_RHO] / S[S_RHO_OLD];
+                                                 Fold f, double *__restrict__ part) {
+    double mean, beta;
+    dir_scalars<FOLD>(c, f, S, first, mean, beta);
     const int j = blockIdx.x * 64 + threadIdx.x;
     double s[1] = {0.};
     for (int i = blockIdx.y * 4 + threadIdx.y; i < c.n1; i += gridDim.y * 4) {
@@ -1926,9 +1982,11 @@ __global__ void __launch_bounds__(64 * SW_WAVES) k_true_rows(TresArgs A) { tres_
 // --- the FP32-vector CG (precision IMPEC_PREC_MIXED32) ----------------------
 // e += alpha d, r -= alpha q in FP32 storage (alpha and the arithmetic in
 // FP64, each result rounded once); partials (r.r, sum r) of the stored r
+template <bool FOLD>
 __global__ void k_cg_update32(CgArgs c, float *__restrict__ e, const float *__restrict__ d, float *__restrict__ r,
-                              const float *__restrict__ qv, const double *__restrict__ S, double *__restrict__ part) {
-    const double alpha = cg_alpha(S);
+                              const float *__restrict__ qv, const double *__restrict__ S, Fold f,
+                              double *__restrict__ part) {
+    const double alpha = update_alpha<FOLD>(f, S);
     const int j = blockIdx.x * 64 + threadIdx.x;
     double s[2] = {0., 0.};
     if (j < c.n2)
@@ -1995,8 +2053,7 @@ __global__ void k_cg_fold32(CgArgs c, double *__restrict__ p, const float *__res
 #endif
 template <class G>
 __device__ __forceinline__ void cg_update2_body(const G &gr_, CgArgs c, double *__restrict__ p, const double *__restrict__ d, double *__restrict__ r,
-                             const double *__restrict__ qv, const double *__restrict__ S, double *__restrict__ part) {
-    const double alpha = cg_alpha(S);
+                             const double *__restrict__ qv, const double alpha, double *__restrict__ part) {
     const int j = gr_.bx() * 64 + threadIdx.x;
     double s[2] = {0., 0.};
     for (int i = gr_.by() * 4 + threadIdx.y; i < c.n1; i += gr_.gy() * 4) {
@@ -2025,9 +2082,11 @@ __device__ __forceinline__ void cg_update2_body(const G &gr_, CgArgs c, double *
         part[RED_BLOCKS + blk] = s[1];
     }
 }
+template <bool FOLD>
 __global__ void k_cg_update2(CgArgs c, double *__restrict__ p, const double *__restrict__ d, double *__restrict__ r,
-                             const double *__restrict__ qv, const double *__restrict__ S, double *__restrict__ part) {
-    cg_update2_body(HwGrid{}, c, p, d, r, qv, S, part);
+                             const double *__restrict__ qv, const double *__restrict__ S, Fold f,
+                             double *__restrict__ part) {
+    cg_update2_body(HwGrid{}, c, p, d, r, qv, update_alpha<FOLD>(f, S), part);
 }
 
 // the finest level's target in the FP64 cycle (3072 waves, 3 per SIMD: 118 and
@@ -2571,6 +2630,37 @@ static DirMvArgs<T> dir_mv_args(impec_ctx *ctx, const LevArgs &a0, const CgArgs 
     return A;
 }
 
+// the direction pass, the update and the sums between and after them, for the
+// three iterations below: dir(fold, part) and upd(fold, part) launch the two
+// passes (fold.n > 0: they form the preceding sums themselves).  Folding saves
+// two launches of one workgroup (4 to 6 us each).  Every workgroup reads the
+// partials for it, so it is done while partials x workgroups stay below
+// IMPEC_FOLD_READS (grids up to about 600^2).
+#ifndef IMPEC_FOLD_READS
+#define IMPEC_FOLD_READS (1l << 20)
+#endif
+template <class Dir, class Upd>
+static int cg_passes(impec_ctx *ctx, const CgArgs &c, int ncycle, int ndir, int wgdir, int nupd, Dir &&dir,
+                     Upd &&upd) {
+    const double inv_n = 1.0 / (double)c.n;
+    const bool fold = ncycle <= FOLD_MAX && ndir <= FOLD_MAX && (long)ncycle * wgdir <= IMPEC_FOLD_READS &&
+                      (long)ndir * nupd <= IMPEC_FOLD_READS;
+    double *dq = ctx->part + (size_t)PART_DQ * RED_BLOCKS;
+    int st;
+    if (!fold)
+        hipLaunchKernelGGL(k_finish_rho, dim3(1), dim3(1024), 0, ctx->stream, ctx->part, ncycle, inv_n, ctx->scal);
+    prof_begin(ctx);
+    dir(Fold{ctx->part, fold ? ncycle : 0, ctx->scal, inv_n}, dq);
+    prof_end(ctx, "cg_dir_matvec");
+    if (!fold && (st = finish_sum(ctx, ndir, 1, S_DQ, PubArgs{nullptr, 0}, PART_DQ))) return st;
+    prof_begin(ctx);
+    upd(Fold{dq, fold ? ndir : 0, ctx->scal, inv_n}, ctx->part + (size_t)PART_RR * RED_BLOCKS);
+    prof_end(ctx, "cg_update");
+    if ((st = finish_sum(ctx, nupd, 2, S_RR, pub_next(ctx), PART_RR))) return st;
+    IMPEC_HIP_CHECK(ctx, hipGetLastError());
+    return IMPEC_OK;
+}
+
 // one CG iteration with the streaming V-cycle (nu = 1) in storage type T
 // (double: plain FP64; float: the FP32 cycle of the mixed-precision solve);
 // the CG vectors, the residual and every reduction stay FP64; d ping-pongs.
@@ -2578,26 +2668,29 @@ static DirMvArgs<T> dir_mv_args(impec_ctx *ctx, const LevArgs &a0, const CgArgs 
 template <typename T>
 static int cg_iteration_fused(impec_ctx *ctx, const LevArgs &a0, const CgArgs &c, bool first, double **dold,
                               double **dnew, bool first_leg_queued = false) {
-    const Level &L0 = ctx->lev[0];
     hipStream_t s = ctx->stream;
     const Grid2 vg = vec_grid(ctx->N1, ctx->N2);
-    const int nwave0 = fused_args<T>(ctx, 0).nwave;
-    const double inv_n = 1.0 / (double)c.n;
     int st;
     if ((st = vcycle_fused<T>(ctx, false, first_leg_queued))) return st;
-    hipLaunchKernelGGL(k_finish_rho, dim3(1), dim3(1024), 0, s, ctx->part, nwave0, inv_n, ctx->scal);
     const DirMvArgs<T> dm = dir_mv_args<T>(ctx, a0, c);
-    prof_begin(ctx);
-    hipLaunchKernelGGL((k_dir_mv<T>), dim3((dm.nwave + SW_WAVES - 1) / SW_WAVES), dim3(64 * SW_WAVES), 0, s, dm, *dold,
-                       *dnew, first ? 1 : 0);
-    prof_end(ctx, "cg_dir_matvec");
-    if ((st = finish_sum(ctx, dm.nwave, 1, S_DQ))) return st;
-    prof_begin(ctx);
-    hipLaunchKernelGGL(k_cg_update2, vg.grid, vg.block, 0, s, c, ctx->p, *dnew, ctx->pr, ctx->pq, ctx->scal,
-                       ctx->part);
-    prof_end(ctx, "cg_update");
-    if ((st = finish_sum(ctx, vg.nblocks, 2, S_RR, pub_next(ctx)))) return st;
-    IMPEC_HIP_CHECK(ctx, hipGetLastError());
+    const dim3 gd((dm.nwave + SW_WAVES - 1) / SW_WAVES), bd(64 * SW_WAVES);
+    st = cg_passes(
+        ctx, c, fused_args<T>(ctx, 0).nwave, dm.nwave, (int)gd.x, vg.nblocks,
+        [&](const Fold &f, double *part) {
+            DirMvArgs<T> A = dm;
+            A.part = part;
+            if (f.n) hipLaunchKernelGGL((k_dir_mv<T, double, true>), gd, bd, 0, s, A, *dold, *dnew, first ? 1 : 0, f);
+            else hipLaunchKernelGGL((k_dir_mv<T, double, false>), gd, bd, 0, s, A, *dold, *dnew, first ? 1 : 0, f);
+        },
+        [&](const Fold &f, double *part) {
+            if (f.n)
+                hipLaunchKernelGGL(k_cg_update2<true>, vg.grid, vg.block, 0, s, c, ctx->p, *dnew, ctx->pr, ctx->pq,
+                                   ctx->scal, f, part);
+            else
+                hipLaunchKernelGGL(k_cg_update2<false>, vg.grid, vg.block, 0, s, c, ctx->p, *dnew, ctx->pr, ctx->pq,
+                                   ctx->scal, f, part);
+        });
+    if (st) return st;
     double *t = *dold;
     *dold = *dnew;
     *dnew = t;
@@ -2611,17 +2704,25 @@ static int cg_iteration_blocks9(impec_ctx *ctx, const CgArgs &c, bool first, dou
     const Grid2 vg = vec_grid(ctx->N1, ctx->N2);
     int st, parts = 0;
     if ((st = mg_ns(ctx) == 2 ? vcycle9<2>(ctx, &parts) : vcycle9<1>(ctx, &parts))) return st;
-    hipLaunchKernelGGL(k_finish_rho, dim3(1), dim3(1024), 0, s, ctx->part, parts, 1.0 / (double)c.n, ctx->scal);
-    prof_begin(ctx);
-    hipLaunchKernelGGL(k_dir_mv9, vg.grid, vg.block, 0, s, op_planes(L0), c, L0.r, *dold, *dnew, ctx->pq, ctx->scal,
-                       first ? 1 : 0, ctx->part);
-    prof_end(ctx, "cg_dir_matvec");
-    if ((st = finish_sum(ctx, vg.nblocks, 1, S_DQ))) return st;
-    prof_begin(ctx);
-    hipLaunchKernelGGL(k_cg_update2, vg.grid, vg.block, 0, s, c, ctx->p, *dnew, ctx->pr, ctx->pq, ctx->scal, ctx->part);
-    prof_end(ctx, "cg_update");
-    if ((st = finish_sum(ctx, vg.nblocks, 2, S_RR, pub_next(ctx)))) return st;
-    IMPEC_HIP_CHECK(ctx, hipGetLastError());
+    st = cg_passes(
+        ctx, c, parts, vg.nblocks, vg.nblocks, vg.nblocks,
+        [&](const Fold &f, double *part) {
+            if (f.n)
+                hipLaunchKernelGGL(k_dir_mv9<true>, vg.grid, vg.block, 0, s, op_planes(L0), c, L0.r, *dold, *dnew, ctx->pq,
+                                   ctx->scal, first ? 1 : 0, f, part);
+            else
+                hipLaunchKernelGGL(k_dir_mv9<false>, vg.grid, vg.block, 0, s, op_planes(L0), c, L0.r, *dold, *dnew,
+                                   ctx->pq, ctx->scal, first ? 1 : 0, f, part);
+        },
+        [&](const Fold &f, double *part) {
+            if (f.n)
+                hipLaunchKernelGGL(k_cg_update2<true>, vg.grid, vg.block, 0, s, c, ctx->p, *dnew, ctx->pr, ctx->pq,
+                                   ctx->scal, f, part);
+            else
+                hipLaunchKernelGGL(k_cg_update2<false>, vg.grid, vg.block, 0, s, c, ctx->p, *dnew, ctx->pr, ctx->pq,
+                                   ctx->scal, f, part);
+        });
+    if (st) return st;
     double *t = *dold;
     *dold = *dnew;
     *dnew = t;
@@ -2636,30 +2737,33 @@ static int cg_iteration_mixed32(impec_ctx *ctx, const LevArgs &a0, const CgArgs 
                                 float **dnew) {
     hipStream_t s = ctx->stream;
     const Grid2 vg = vec_grid(ctx->N1, ctx->N2);
-    const int nwave0 = fused_args<float>(ctx, 0).nwave;
-    const double inv_n = 1.0 / (double)c.n;
     int st;
     if ((st = vcycle_fused<float>(ctx, true))) return st;
-    hipLaunchKernelGGL(k_finish_rho, dim3(1), dim3(1024), 0, s, ctx->part, nwave0, inv_n, ctx->scal);
     const DirMvArgs<float> d64 = dir_mv_args<float>(ctx, a0, c, IMPEC_DM_WAVES_F32);
     DirMvArgs<float, float> dm;
     memset(&dm, 0, sizeof(dm));
     dm.L = d64.L; dm.c = d64.c; dm.x0 = d64.x0;
     dm.d0 = ctx->pd32; dm.d1 = ctx->pz32; dm.q = ctx->pq32;
     dm.fx32 = ctx->fx32; dm.fy32 = ctx->fy32;
-    dm.S = d64.S; dm.part = d64.part;
+    dm.S = d64.S;
     dm.R = d64.R; dm.nstrip = d64.nstrip; dm.nwave = d64.nwave;
-    prof_begin(ctx);
-    hipLaunchKernelGGL((k_dir_mv<float, float>), dim3((dm.nwave + SW_WAVES - 1) / SW_WAVES), dim3(64 * SW_WAVES), 0,
-                       s, dm, *dold, *dnew, first ? 1 : 0);
-    prof_end(ctx, "cg_dir_matvec");
-    if ((st = finish_sum(ctx, dm.nwave, 1, S_DQ))) return st;
-    prof_begin(ctx);
-    hipLaunchKernelGGL(k_cg_update32, vg.grid, vg.block, 0, s, c, ctx->pe32, *dnew, ctx->pr32, ctx->pq32, ctx->scal,
-                       ctx->part);
-    prof_end(ctx, "cg_update");
-    if ((st = finish_sum(ctx, vg.nblocks, 2, S_RR, pub_next(ctx)))) return st;
-    IMPEC_HIP_CHECK(ctx, hipGetLastError());
+    const dim3 gd((dm.nwave + SW_WAVES - 1) / SW_WAVES), bd(64 * SW_WAVES);
+    st = cg_passes(
+        ctx, c, fused_args<float>(ctx, 0).nwave, dm.nwave, (int)gd.x, vg.nblocks,
+        [&](const Fold &f, double *part) {
+            dm.part = part;
+            if (f.n) hipLaunchKernelGGL((k_dir_mv<float, float, true>), gd, bd, 0, s, dm, *dold, *dnew, first ? 1 : 0, f);
+            else hipLaunchKernelGGL((k_dir_mv<float, float, false>), gd, bd, 0, s, dm, *dold, *dnew, first ? 1 : 0, f);
+        },
+        [&](const Fold &f, double *part) {
+            if (f.n)
+                hipLaunchKernelGGL(k_cg_update32<true>, vg.grid, vg.block, 0, s, c, ctx->pe32, *dnew, ctx->pr32,
+                                   ctx->pq32, ctx->scal, f, part);
+            else
+                hipLaunchKernelGGL(k_cg_update32<false>, vg.grid, vg.block, 0, s, c, ctx->pe32, *dnew, ctx->pr32,
+                                   ctx->pq32, ctx->scal, f, part);
+        });
+    if (st) return st;
     float *t = *dold;
     *dold = *dnew;
     *dnew = t;
@@ -3247,7 +3351,7 @@ __global__ void kb_update2(const Upd2Rec *__restrict__ tab, const int *__restric
     batch_for(tab, start, nmem, [&](const auto &R, const VGrid &G) {
         if (!in_state(R.S, need)) return;
         const bool odd = ((long long)R.S[S_EITS]) & 1;
-        cg_update2_body(G, R.c, R.p, odd ? R.d0 : R.d1, R.r, R.q, R.S, R.part);
+        cg_update2_body(G, R.c, R.p, odd ? R.d0 : R.d1, R.r, R.q, cg_alpha(R.S), R.part);
     });
 }
 // after the first residual: iterate unless converged (solve_cg's loop entry)
@@ -3431,13 +3535,15 @@ __global__ void __launch_bounds__(64 * SW_WAVES) kp_dir_mv(const DirMvArgs<T> *_
         const DirMvArgs<T> &A = tab[m];
         const bool odd = ((long long)A.S[S_EITS]) & 1;
         const int first = A.S[S_ESINCE] == 0.;
-        dir_mv_body<T>(A, odd ? A.d1 : A.d0, odd ? A.d0 : A.d1, first, loc);
+        double mean, beta;
+        dir_scalars<false>(A.c, Fold{}, A.S, first, mean, beta);
+        dir_mv_body<T>(A, odd ? A.d1 : A.d0, odd ? A.d0 : A.d1, first, loc, mean, beta);
     });
 }
 __global__ void kp_update2(const Upd2Rec *__restrict__ tab, ActList act) {
     act_for(tab, act, [&](const Upd2Rec &R, const VGrid &G) {
         const bool odd = ((long long)R.S[S_EITS]) & 1;
-        cg_update2_body(G, R.c, R.p, odd ? R.d0 : R.d1, R.r, R.q, R.S, R.part);
+        cg_update2_body(G, R.c, R.p, odd ? R.d0 : R.d1, R.r, R.q, cg_alpha(R.S), R.part);
     });
 }
 __global__ void kp_cg_init(const CgInitRec *__restrict__ tab, ActList act) {
