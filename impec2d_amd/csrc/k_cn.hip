@@ -81,6 +81,38 @@ __device__ __forceinline__ void yface_tensor(const CnConst &k, double ub, double
     d22 = x22;
 }
 
+// The two tensors with phi alpha / |u| formed from a reciprocal square root (the
+// hardware estimate and two Newton steps, y' = y + y (1/2 - (q/2) y^2), to about
+// an ulp) in place of a square root and two divisions: for the solver's own
+// operator applications, the s- and p-launches, whose rounding the true
+// residual with the exact tensors (CN_R, CN_RX) checks before a solve ends.  Those
+// launches are limited by instruction issue as much as by bytes: at 4096^2 the
+// s-launch takes 168.5 us against 184.8 and the p-launch 295 against 304, at
+// 1024^2 20.5 against 25.7 and 28.6 against 33.2; the true residuals reached are
+// the same.  Outside the range where the steps neither overflow nor lose bits, and for
+// speed zero, the exact ones.
+__device__ __forceinline__ bool rsqrt_fast(double q, double &y) {
+    const double h = 0.5 * q;
+    y = __builtin_amdgcn_rsq(q);
+    y = fma(y, fma(-(h * y), y, 0.5), y);
+    y = fma(y, fma(-(h * y), y, 0.5), y);
+    return q >= 0x1p-900 && q <= 0x1p+900;
+}
+__device__ __forceinline__ void xface_tensor_fast(const CnConst &k, double uu, double vb, double &d11, double &d12) {
+    const double u2 = uu * uu, v2 = vb * vb;
+    double y;
+    if (__builtin_expect(!rsqrt_fast(u2 + v2, y), 0)) {
+        xface_tensor(k, uu, vb, d11, d12);
+        return;
+    }
+    const double fl = k.phal * y, ft = k.phat * y;
+    d11 = fma(fl, u2, fma(ft, v2, k.phdm));
+    d12 = (fl - ft) * (uu * vb);
+}
+__device__ __forceinline__ void yface_tensor_fast(const CnConst &k, double ub, double vv, double &d22, double &d21) {
+    xface_tensor_fast(k, vv, ub, d22, d21);   // the same with the two components exchanged
+}
+
 // the eight face tensors around cell (i, j) (west / east x-faces, south /
 // north y-faces) from the ghost-filled u and v, with the four-point averages
 // of SetupDiffusionTensorF/G in their summation order
@@ -290,6 +322,7 @@ __device__ __forceinline__ double cn_apply(const double a[9], double Y0, double 
 // of face m (from u and v of rows m-1 and m) and the y-face tensors of row m-1
 // (from u of rows m-1 and m), the four-point averages of cell_tensors in its
 // summation order; cell(...) then gives row m-1's eight tensors
+template <bool FAST>
 struct FaceStream {
     double uprev, vprev, uprev_l, vprev_n;   // u, v of row m-1 and their lane shifts
     double f11a = 0., f12a = 0., f11b = 0., f12b = 0.;   // x-faces m-1 and m
@@ -301,9 +334,11 @@ struct FaceStream {
         const double um_l = lane_prev(um), vm_n = lane_next(vm);
         double e11, e12;
         const double vb = 1. / 4 * (vprev_n + vm_n + vprev + vm);
-        xface_tensor(k, um, vb, e11, e12);
+        if (FAST) xface_tensor_fast(k, um, vb, e11, e12);
+        else xface_tensor(k, um, vb, e11, e12);
         const double ub = 1. / 4 * (um_l + um + uprev_l + uprev);
-        yface_tensor(k, ub, vprev, g22, g21);
+        if (FAST) yface_tensor_fast(k, ub, vprev, g22, g21);
+        else yface_tensor(k, ub, vprev, g22, g21);
         uprev = um; vprev = vm; uprev_l = um_l; vprev_n = vm_n;
         f11a = f11b; f12a = f12b; f11b = e11; f12b = e12;
     }
@@ -383,7 +418,7 @@ __global__ void __launch_bounds__(64 * CNS_WAVES) k_cn_stream(CnArgs A) {
     // windows: the operator's input y of rows m-2, m-1, m; the vector of row
     // m-1 (s or p) and r0 of row m-1
     double Y0 = 0., Y1 = 0., Y2 = 0.;
-    FaceStream fs;
+    FaceStream<MODE == CN_S> fs;
     fs.start(vel(A.u, mstart - 1), vel(A.v, mstart - 1));
     double wprev = 0., r0prev = 0., bprev = 0.;
     double s0 = 0., s1 = 0., s2 = 0., s3 = 0., s4 = 0.;
@@ -540,7 +575,7 @@ __global__ void __launch_bounds__(64 * CN_WAVES, IMPEC_CNP_MIN_WAVES) k_cn_pstep
     double YP0 = 0., YP1 = 0., YP2 = 0.;   // p'/D of rows m-3, m-2, m-1
     double sprev = 0., vprev = 0., dprev = 0.;   // s, v and 1/D of row m-1
     double aprev[9] = {};                  // coefficients of row m-2
-    FaceStream fs;
+    FaceStream<true> fs;   // as the s-launch, whose s and t it forms again
     fs.start(vel(A.u, mstart - 1), vel(A.v, mstart - 1));
     double s0 = 0., s1 = 0.;
     for (int mb = mstart; mb < mstop; mb += PF) {
@@ -647,7 +682,7 @@ __global__ void __launch_bounds__(64 * CNZ_WAVES) k_cn_start(CnArgs A, const dou
     double Y0 = 0., Y1 = 0., Y2 = 0.;      // b/D of rows m-3, m-2, m-1
     double bprev = 0.;                     // r0 = b rounded to FP32, of row m-2
     double aprev[9] = {};                  // coefficients of row m-2
-    FaceStream fs;
+    FaceStream<false> fs;
     fs.start(vel(A.u, mstart - 1), vel(A.v, mstart - 1));
     double s0 = 0., s1 = 0., s2 = 0.;
     for (int mb = mstart; mb < mstop; mb += PF) {
