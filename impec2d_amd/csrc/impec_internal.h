@@ -76,6 +76,13 @@ enum { EST_DONE = 0, EST_ITER = 1, EST_CHECK = 2 };
 #ifndef IMPEC_STALL_ITS
 #define IMPEC_STALL_ITS 20
 #endif
+// ... or, once its norm is below the rounding floor that the solve before this
+// one met, in IMPEC_STALL_FLOOR_ITS: there the wait for 20 buys nothing (141^2
+// cells, eps 1e-14: the true residual is 2.1e-12 after 18 iterations and 2.1e-12
+// after 38).
+#ifndef IMPEC_STALL_FLOOR_ITS
+#define IMPEC_STALL_FLOOR_ITS 5
+#endif
 #ifndef IMPEC_STALL_GATE
 #define IMPEC_STALL_GATE 4.0
 #endif

@@ -2876,6 +2876,7 @@ static int solve_cg(impec_ctx *ctx, int *its_out, double *relres_out) {
     int its = 0, status = IMPEC_OK;
     double relres = 0., rr = 0.;
     double floor_rel = 0., tol_eff = tol;   // the true residual's rounding floor, max(tol, floor)
+    const double floor_hint = ctx->stats.last_relres_floor;   // that of the solve before (0: none yet)
     double *dold = ctx->pd, *dnew = ctx->pz;
     float *dold32 = ctx->pd32, *dnew32 = ctx->pz32;
     double rr_ref = 0.;   // FP64 residual norm^2 at the FP32 recursion's last restart
@@ -2979,7 +2980,8 @@ static int solve_cg(impec_ctx *ctx, int *its_out, double *relres_out) {
                 if (rr <= 0.25 * rr_mark) {
                     rr_mark = rr;
                     stall = 0;
-                } else if (++stall >= IMPEC_STALL_ITS && rr == rr && !(rr <= tol * tol * bb)) {
+                } else if (++stall >= (rr <= floor_hint * floor_hint * bb ? IMPEC_STALL_FLOOR_ITS : IMPEC_STALL_ITS) &&
+                           rr == rr && !(rr <= tol * tol * bb)) {
                     // the pinned system's true residual and floor (p moves by a
                     // constant in the consistent phase, its pinned value is kept
                     // in the elimination phase: the recursion is unchanged)
