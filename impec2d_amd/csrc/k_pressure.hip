@@ -676,10 +676,41 @@ __global__ void k_sum(CgArgs c, const double *__restrict__ x0, double *__restric
     if (tid_linear() == 0) part[blockIdx.x] = s[0];
 }
 
+// The preconditioner of the eliminated formulation.  With the pinned row and
+// column taken out the operator is regular, but its smallest eigenvalue, of a
+// nearly constant vector, goes with the coupling of one cell to its neighbours,
+// and the V-cycle of the Neumann operator (output less its mean) says nothing
+// about constants: CG found that vector by itself, in about 20 iterations in
+// which the residual wandered around its start.  The missing part is a one-
+// vector correction z += v (v.r) / (v.A v), v = 1 off the pinned cell, which is
+// a constant added to the V-cycle's output: v.A v = -sum of the neighbours'
+// coefficients towards the pinned cell (S_PINSUM, k_pin_sum), v.r = sum r.
+// Iterations to 1e-10 at nu = 2/3: 100 x 50 cells 28 -> 19, 300 x 290 30 -> 18,
+// 500 x 260 35 -> 21; nu = 0, 100 x 50: 97 -> 62.
+__device__ __forceinline__ double pin_shift(int shift, const double *__restrict__ S) {
+    return shift ? 0. : S[S_RSUM] * S[S_PINSUM];
+}
+template <bool DIAG>
+__global__ void k_pin_sum(LevArgs L, int pi, int pj, double *__restrict__ S) {
+    const int dI[9] = {0, -1, -1, 0, 1, 1, 1, 0, -1}, dJ[9] = {0, 0, -1, -1, -1, 0, 1, 1, 1};
+    double s = 0.;
+#pragma unroll
+    for (int q = 1; q < 9; q++) {
+        const int i = pi + dI[q], j = pj + dJ[q];
+        if (i < 0 || j < 0 || i >= L.g.n1 || j >= L.g.n2) continue;
+        double a[9];
+        op_row_L<DIAG>(L, i, j, a);
+#pragma unroll
+        for (int k = 1; k < 9; k++)
+            if (dI[q] + dI[k] == 0 && dJ[q] + dJ[k] == 0) s -= a[k];
+    }
+    S[S_PINSUM] = s != 0. && isfinite(s) ? 1. / s : 0.;
+}
+
 // z = x0 - mean(x0) (pin entry zeroed in the eliminated formulation); r.z partials
 __global__ void k_cg_z(CgArgs c, const double *__restrict__ x0, const double *__restrict__ r, double *__restrict__ z,
                        const double *__restrict__ S, double *__restrict__ part) {
-    const double mean = S[S_ZSUM] / (double)c.n;
+    const double mean = S[S_ZSUM] / (double)c.n - pin_shift(c.shift, S);
     double s[1] = {0.};
     for (long id = (long)blockIdx.x * blockDim.x + threadIdx.x; id < c.n; id += (long)gridDim.x * blockDim.x) {
         int i, j;
@@ -1605,7 +1636,8 @@ static int top_level(const impec_ctx *ctx) {
 
 // sums of the V-cycle output and rho = r.z with z = x0 - mean(x0)
 template <class G>
-__device__ __forceinline__ void finish_rho_body(const G &gr_, const double *__restrict__ part, int nblocks, double inv_n, double *__restrict__ S) {
+__device__ __forceinline__ void finish_rho_body(const G &gr_, const double *__restrict__ part, int nblocks, double inv_n, double *__restrict__ S,
+                                                int shift = 1) {
     double v[2];
     strided_combine_nv<RED_SUM, 2>(part, RED_BLOCKS, nblocks, v);
     block_reduce<RED_SUM, 2>(v);
@@ -1613,11 +1645,12 @@ __device__ __forceinline__ void finish_rho_body(const G &gr_, const double *__re
         S[S_ZSUM] = v[0];
         S[S_RX] = v[1];
         S[S_RHO_OLD] = S[S_RHO];
-        S[S_RHO] = v[1] - v[0] * inv_n * S[S_RSUM];
+        S[S_RHO] = v[1] - (v[0] * inv_n - pin_shift(shift, S)) * S[S_RSUM];
     }
 }
-__global__ void k_finish_rho(const double *__restrict__ part, int nblocks, double inv_n, double *__restrict__ S) {
-    finish_rho_body(HwGrid{}, part, nblocks, inv_n, S);
+__global__ void k_finish_rho(const double *__restrict__ part, int nblocks, double inv_n, double *__restrict__ S,
+                             int shift) {
+    finish_rho_body(HwGrid{}, part, nblocks, inv_n, S, shift);
 }
 
 // tiled 2-D launch shape for the level-0 vector kernels: 64 x 4 threads,
@@ -1674,15 +1707,17 @@ struct Fold {
 constexpr int PART_CYCLE = 0, PART_DQ = 2, PART_RR = 3;
 static_assert(PART_RR + 2 <= PART_VECS, "vectors of the CG's partial sums");
 
-// mean of the V-cycle's output and beta of the direction update
+// mean of the V-cycle's output (for the eliminated formulation: less the constant
+// of pin_shift) and beta of the direction update
 template <bool FOLD>
 __device__ __forceinline__ void dir_scalars(const CgArgs &c, const Fold &f, const double *__restrict__ S, int first,
                                             double &mean, double &beta) {
     if constexpr (FOLD) {
         double v[2];
         fold_sums<2>(f.part, RED_BLOCKS, f.n, v);
-        const double rho = v[1] - v[0] * f.inv_n * S[S_RSUM];
-        mean = v[0] / (double)c.n;
+        const double shift = pin_shift(c.shift, S);
+        const double rho = v[1] - (v[0] * f.inv_n - shift) * S[S_RSUM];
+        mean = v[0] / (double)c.n - shift;
         beta = first ? 0. : rho / S[S_RHO];   // S_RHO: the previous iteration's until this one's update
         if (tid_linear() == 0 && blockIdx.x == 0 && blockIdx.y == 0) {
             f.S[S_ZSUM] = v[0];
@@ -1690,7 +1725,7 @@ __device__ __forceinline__ void dir_scalars(const CgArgs &c, const Fold &f, cons
             f.S[S_RHO_NEXT] = rho;
         }
     } else {
-        mean = S[S_ZSUM] / (double)c.n;
+        mean = S[S_ZSUM] / (double)c.n - pin_shift(c.shift, S);
         beta = first ? 0. : S[S_RHO] / S[S_RHO_OLD];
     }
 }
@@ -2648,7 +2683,8 @@ static int cg_passes(impec_ctx *ctx, const CgArgs &c, int ncycle, int ndir, int 
     double *dq = ctx->part + (size_t)PART_DQ * RED_BLOCKS;
     int st;
     if (!fold)
-        hipLaunchKernelGGL(k_finish_rho, dim3(1), dim3(1024), 0, ctx->stream, ctx->part, ncycle, inv_n, ctx->scal);
+        hipLaunchKernelGGL(k_finish_rho, dim3(1), dim3(1024), 0, ctx->stream, ctx->part, ncycle, inv_n, ctx->scal,
+                           c.shift);
     prof_begin(ctx);
     dir(Fold{ctx->part, fold ? ncycle : 0, ctx->scal, inv_n}, dq);
     prof_end(ctx, "cg_dir_matvec");
@@ -2883,6 +2919,7 @@ static int solve_cg(impec_ctx *ctx, int *its_out, double *relres_out) {
     int restarts_all = 0, elim_its = 0;
     for (int phase = ctx->symmetric ? 0 : 1; phase < 2; phase++) {
         c.shift = phase == 0;
+        if (!c.shift) hipLaunchKernelGGL(k_pin_sum<DIAG>, dim3(1), dim3(1), 0, s, a0, c.pin_i, c.pin_j, ctx->scal);
         const int its_at_start = its;
         // the FP32-vector CG runs the consistent phase; the elimination phase, a
         // short continuation at the FP64 rounding floor of a worse-conditioned

@@ -59,3 +59,46 @@ def test_block_cycle_iteration_counts(gpu_lib, n1, n2):
         g.close()
     assert abs(its[0] - its[1]) <= 1, its
     assert rel_err(ps[0], ps[1]) < 1e-8
+
+
+@pytest.mark.parametrize("n1,n2,nu,aniso", [(100, 50, 2 / 3, False), (64, 64, 0.5, True), (150, 145, 1 / 3, False),
+                                            (9, 5, 2 / 3, False), (3, 3, 2 / 3, True)])
+def test_eliminated_formulation_needs_no_search_for_the_constant(gpu_lib, n1, n2, nu, aniso):
+    """dx != dy or anisotropic K (the pinned row and column eliminated): the
+    preconditioner's constant makes CG start at once.  Without it these solves
+    took 21 to 28 iterations, about ten of them for the nearly constant vector; a
+    consistent system of the same size takes 10 to 15.  Both cycles agree, as in
+    test_block_cycle_iteration_counts."""
+    p = params(N1=n1, N2=n2, nu=nu, mu_inj=1 / 20., eps=1e-10)
+    rng = np.random.default_rng(n1)
+    K11 = np.exp(0.3 * rng.standard_normal((n1 + 4, n2 + 4)))
+    K22 = np.exp(0.3 * rng.standard_normal((n1 + 4, n2 + 4))) if aniso else None
+    its, ps = [], []
+    for variant in (0, 1):
+        o, g = pair(p, K11, K22, mg_variant=variant)
+        g.set_source(o.source())
+        g.set_concentration(smooth_c(o))
+        n, _ = g.pressure_solve()
+        its.append(n)
+        ps.append(o.interior(g.get_pressure()).copy())
+        assert g.stats().last_elim_its == n
+        g.close()
+    assert max(its) <= 20 and abs(its[0] - its[1]) <= 1, its
+    assert rel_err(ps[0], ps[1]) < 1e-8
+
+
+def test_tolerance_below_the_floor_does_not_wait_for_the_stall(gpu_lib):
+    """eps = 1e-14 lies below the rounding floor: once a solve has met the floor,
+    the next ones stop within 5 iterations of reaching it instead of 20, at a
+    residual still below it."""
+    p = params(N1=141, N2=141, stype=0, x_ub=2 ** 0.5, y_ub=2 ** 0.5, nu=2 / 3, mu_res=41.0, mu_inj=1.0, eps=1e-14)
+    o, g = pair(p)
+    g.set_source(o.source("circle"))
+    g.set_concentration(smooth_c(o))
+    g.fill_boundaries()
+    first, _ = g.pressure_solve()
+    again, _ = g.pressure_solve()
+    s = g.stats()
+    assert first - 20 <= again <= first - 10, (first, again)
+    assert s.last_relres <= s.last_relres_floor
+    g.close()
