@@ -181,6 +181,9 @@ struct impec_ctx {
     // correction since the last reliable update, direction pair, matvec, and
     // FP32 copies of fx / fy
     float *pr32, *pe32, *pd32, *pz32, *pq32, *fx32, *fy32;
+    // the 5-point bottom's coefficients per solve (mg_block.h: 16 doubles of the
+    // coarsest level's solution operator, then BOT_IMG values), FP64 and FP32 cycle
+    char *bot_img, *bot_img32;
     double *op9_inv;           // coarsest level's solution operator of the 9-point cycle
     double *scal;              // device scalars (Scal)
     double *part;              // reduction partials

@@ -960,6 +960,9 @@ int pressure_setup_levels(impec_ctx *ctx) {
         hipMemset(*vecs[k], 0, bytes0);
     }
     if (ctx->P.nu != 1. && blocks9_ok(ctx)) op9_alloc(ctx);
+    if (hipMalloc(&ctx->bot_img, bot_img_bytes<double>()) != hipSuccess)
+        return set_error(ctx, IMPEC_ENOMEM, "multigrid bottom allocation failed");
+    hipMemset(ctx->bot_img, 0, bot_img_bytes<double>());
     return IMPEC_OK;
 }
 
@@ -976,6 +979,9 @@ void pressure_free_levels(impec_ctx *ctx) {
     hipFree(ctx->fx); hipFree(ctx->fy);
     if (ctx->op9_inv) hipFree(ctx->op9_inv);
     ctx->op9_inv = nullptr;
+    if (ctx->bot_img) hipFree(ctx->bot_img);
+    if (ctx->bot_img32) hipFree(ctx->bot_img32);
+    ctx->bot_img = ctx->bot_img32 = nullptr;
     float **v32[7] = {&ctx->pr32, &ctx->pe32, &ctx->pd32, &ctx->pz32, &ctx->pq32, &ctx->fx32, &ctx->fy32};
     for (float **v : v32) {
         if (*v) hipFree(*v);
@@ -1608,6 +1614,10 @@ template <typename T, bool NINE>
 __global__ void __launch_bounds__(BOTTOM_THREADS) k_mg_bottom(BottomArgs<T> A) {
     __shared__ BotShared<T, NINE> sh;
     mg_bottom_body<T, NINE>(A, sh);
+}
+template <typename T>
+__global__ void __launch_bounds__(1024) k_bot5_setup(BottomArgs<T> A) {
+    bot5_setup_body<T>(A, blockIdx.x, const_cast<T *>(A.img), const_cast<double *>(A.inv));
 }
 static int bottom_threads(int d0) { return d0 == 0 ? BOTTOM_THREADS : 256; }
 
@@ -2270,7 +2280,20 @@ static BottomArgs<T> bottom_args(impec_ctx *ctx, int lb) {
     A.ldo = B.ld;
     A.ns = mg_ns(ctx);
     A.S = ctx->scal;
+    char *img = std::is_same<T, float>::value ? ctx->bot_img32 : ctx->bot_img;
+    A.inv = (double *)img;
+    A.img = (T *)(img + 16 * sizeof(double));
     return A;
+}
+
+// the bottom's coefficients for the current mobilities
+template <typename T>
+static int bottom_setup(impec_ctx *ctx) {
+    const int lb = bottom_level(ctx);
+    if (lb <= 0) return IMPEC_OK;
+    hipLaunchKernelGGL(k_bot5_setup<T>, dim3(BOT_DEPTHS), dim3(1024), 0, ctx->stream, bottom_args<T>(ctx, lb));
+    IMPEC_HIP_CHECK(ctx, hipGetLastError());
+    return IMPEC_OK;
 }
 
 // whether level l runs the tile legs of mg_block.h instead of the streaming ones:
@@ -2538,6 +2561,11 @@ static int mixed_alloc(impec_ctx *ctx) {
                 return set_error(ctx, IMPEC_ENOMEM, "mixed-precision level %d allocation failed", l);
             hipMemset(*arrs[k], 0, bytes);
         }
+    }
+    if (!ctx->bot_img32) {
+        if (hipMalloc(&ctx->bot_img32, bot_img_bytes<float>()) != hipSuccess)
+            return set_error(ctx, IMPEC_ENOMEM, "mixed-precision multigrid bottom allocation failed");
+        hipMemset(ctx->bot_img32, 0, bot_img_bytes<float>());
     }
     return IMPEC_OK;
 }
@@ -2857,6 +2885,7 @@ static int solve_cg(impec_ctx *ctx, int *its_out, double *relres_out) {
     if (st) return st;
     if (F32 && (st = mixed_convert(ctx, 1))) return st;
     if (DIAG && FUSED && (st = op9_assemble(ctx))) return st;
+    if (!DIAG && FUSED && (st = bottom_setup<T>(ctx))) return st;
     // the FP32-vector CG with reliable FP64 updates (streaming 5-point path)
     const bool m32 = std::is_same<T, float>::value && FUSED && !DIAG && ctx->P.precision == IMPEC_PREC_MIXED32;
     const Level &L0 = ctx->lev[0];
@@ -3369,8 +3398,13 @@ __global__ void __launch_bounds__(LEG5_P *LEG5_P) kb_mg5_up(const Leg5Args<T> *_
     leg5_up_body<LEG5_P, NS, T>(A, blockIdx.x - start[m], sm);
 }
 template <typename T>
+__global__ void __launch_bounds__(1024) kb_bot5_setup(const BottomArgs<T> *__restrict__ tab) {
+    const BottomArgs<T> &A = tab[blockIdx.y];
+    bot5_setup_body<T>(A, blockIdx.x, const_cast<T *>(A.img), const_cast<double *>(A.inv));
+}
+template <typename T>
 __global__ void __launch_bounds__(BOTTOM_THREADS) kb_mg_bottom(const BottomArgs<T> *__restrict__ tab, int need) {
-    const BottomArgs<T> &A = tab[blockIdx.x];
+    const BottomArgs<T> A = tab[blockIdx.x];
     if (!in_state(A.S, need)) return;
     __shared__ BotShared<T, false> sh;
     mg_bottom_body<T, false>(A, sh);
@@ -3930,6 +3964,11 @@ int ens_solve_begin(impec_ensemble *e) {
     for (int l = 1; l < t->lmax; l++) ENS_CHECK(e, launch_b(kb_coarsen_w, t->coarsen[l], blk, s));
     if (t->mixed)
         for (int l = 0; l < t->lmax; l++) ENS_CHECK(e, launch_b(kb_to_f32, t->tof32[l], blk, s));
+    if (t->mixed && t->l32.bottom.nmem)
+        hipLaunchKernelGGL(kb_bot5_setup<float>, dim3(BOT_DEPTHS, t->l32.bottom.nmem), dim3(1024), 0, s, t->l32.bottom.tab);
+    if (!t->mixed && t->l64.bottom.nmem)
+        hipLaunchKernelGGL(kb_bot5_setup<double>, dim3(BOT_DEPTHS, t->l64.bottom.nmem), dim3(1024), 0, s, t->l64.bottom.tab);
+    ENS_CHECK(e, hipGetLastError());
     ENS_CHECK(e, launch_b(kb_faces, t->faces, blk, s));
     ENS_CHECK(e, launch_b(kb_zero_p, t->zero, dim3(256), s));
     ENS_CHECK(e, launch_b(kb_cg_init, t->init, dim3(256), s, -1));

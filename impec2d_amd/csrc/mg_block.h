@@ -551,16 +551,19 @@ __device__ __forceinline__ void make_co5(const T (&w)[4], const T (&wu)[2], cons
 // to the coarsest and back up in one workgroup.  Depth D holds a level of at
 // most 64 >> D cells a side on (32 >> D)^2 threads; from depth 2 on one wave
 // does the work and needs no workgroup barrier.  The coarsest level (at most
-// 2 x 2 cells) has depth 5; its solution operator is formed by the second wave
-// while the first one works its way down.
+// 2 x 2 cells) has depth 5; its solution operator is formed once per solve.
 //
 // One workgroup is bound by latency: LDS round trips, dependent FP64 chains and
 // the fetch of its own code, which every launch starts without.  So the depths
 // share one loop body (the planes of all depths have one pitch) instead of an
 // unrolled copy each, all loads of the level data are issued together, and what
-// is needed again on the way up is kept in LDS.  FP64, 5-point: 28.9 us from
-// 64^2, 19.7 us from 32^2 (one cell per thread and a barrier per phase on every
-// level: 21.5 us from 32^2, plus 19 us for the two legs of the 64^2 level).
+// is needed again on the way up is kept in LDS.  The 5-point coefficients are
+// formed once per solve (k_bot5_setup, 6 us): forming them from w on both ways of
+// every V-cycle took a third of the bottom.  FP64, 5-point, kernel trace: 20.3 us
+// from 64^2 (28.9 with the coefficients formed in the cycle), 14.5 us from 32^2
+// (19.7); with one cell per thread and a barrier per phase on every level 21.5 us
+// from 32^2, plus 19 us for the two legs of the 64^2 level.  A step of the 1024^2
+// quarter five-spot: 2.46 -> 2.36 ms, of the 64^2 one 0.79 -> 0.74.
 // 9-point: 24 us from 36^2, in place of about 100 launches of 4.5 us.  The
 // 9-point coefficients of the deeper levels kept in LDS measured slower (27.6 us:
 // the copy costs more than the cached reads).
@@ -587,10 +590,18 @@ __device__ __forceinline__ int bot_rhs_at(int d) {   // d >= 1
 
 template <typename T>
 struct BotLev {
-    const T *w;          // mobility quantity at cell (0, 0), pitch ldw (5-point)
+    const T *w;          // mobility quantity at cell (0, 0), pitch ldw (5-point: k_bot5_setup)
     OpPlanes<T> A;       // assembled operator (9-point)
     int ldw;
 };
+// The 5-point coefficients of the bottom's levels, formed once per solve
+// (k_bot5_setup): coefficient q of a block at q * blocks + block, for depth 0 and
+// then, as they go into LDS, for depths 1..4 (block t of depth d at
+// bot_rhs_at(d) / 4 + t).
+constexpr int BOT_CO = 16, BOT_SMALL = 256 + 64 + 16 + 4 + 1;
+constexpr int BOT_IMG = BOT_CO * (1024 + BOT_SMALL);
+template <typename T>
+constexpr size_t bot_img_bytes() { return 16 * sizeof(double) + BOT_IMG * sizeof(T); }
 // The sizes and spacings of the deeper levels follow from the first one's
 // (halved, rounded up; spacings doubled): reading them per level would be a
 // cold scalar load in every depth's chain.
@@ -600,7 +611,8 @@ struct BottomArgs {
     int n1, n2;                    // first level
     double cx, cy;                 // its 1 / dx^2, 1 / dy^2
     BotLev<T> lev[BOT_DEPTHS];
-    const double *inv;             // coarsest level's solution operator (9-point: k_op9_coarsest)
+    const double *inv;             // coarsest level's solution operator
+    const T *img;                  // 5-point coefficients (BOT_IMG values)
     const T *b;                    // right-hand side of the first level at (0, 0)
     T *out;                        // its solution
     int ldb, ldo;
@@ -620,23 +632,22 @@ struct BotSize {   // of the level at depth d
     }
 };
 
-// LDS: the 5-point bottom keeps w of every depth, the 9-point one reads its
-// operator from the caches
+// LDS: the 5-point bottom keeps the coefficients of depths 1..4, the 9-point one
+// reads its operator from the caches
 template <typename T, bool NINE>
 struct alignas(16) BotShared {
     T x[BotGeo::CELLS], r[BotResGeo::CELLS], b[BOT_RHS];   // cleared at the start
-    T w[NINE ? 1 : BotGeo::CELLS];
+    T co[NINE ? 4 : BOT_CO * BOT_SMALL];
     double inv[16];
     static constexpr int CLEAR16 = (BotGeo::CELLS + BotResGeo::CELLS + BOT_RHS) * (int)sizeof(T) / 16;
 };
 
-// the coarsest level of N1 x N2 <= 2 x 2 cells: column k (lane k) of the
-// solution operator of the singular Neumann system bordered by the zero-mean
-// condition, [A 1; 1^T 0][x; l] = [b; 0], A with the legs' faces; FP64 in
-// both precisions
+// the coarsest level of N1 x N2 <= 2 x 2 cells: column k of the solution operator
+// of the singular Neumann system bordered by the zero-mean condition,
+// [A 1; 1^T 0][x; l] = [b; 0], A with the legs' faces; FP64 in both precisions
 template <int N1, int N2, typename T>
-__device__ __forceinline__ void bot5_inverse(const T *w, T cx, T cy, int hm, int k, double *inv) {
-    constexpr int n = N1 * N2, m = n + 1, PL = BotGeo::PLANE;
+__device__ __forceinline__ void bot5_inverse(const T *w, int ld, T cx, T cy, int hm, int k, double *inv) {
+    constexpr int n = N1 * N2, m = n + 1;
     double M[m][m + 1];
 #pragma unroll
     for (int r = 0; r < m; r++)
@@ -649,11 +660,11 @@ __device__ __forceinline__ void bot5_inverse(const T *w, T cx, T cy, int hm, int
         M[b][a] += (double)f;
     };
     constexpr int C01 = N2 > 1 ? 1 : 0, C10 = N1 > 1 ? N2 : 0, C11 = N1 > 1 && N2 > 1 ? 3 : 0;
-    if constexpr (N1 > 1) link(0, C10, cx * face_mob_pc(w[0], w[2 * PL], hm));
-    if constexpr (N2 > 1) link(0, C01, cy * face_mob_pc(w[0], w[PL], hm));
+    if constexpr (N1 > 1) link(0, C10, cx * face_mob_pc(w[0], w[ld], hm));
+    if constexpr (N2 > 1) link(0, C01, cy * face_mob_pc(w[0], w[1], hm));
     if constexpr (N1 > 1 && N2 > 1) {
-        link(C01, C11, cx * face_mob_pc(w[PL], w[3 * PL], hm));
-        link(C10, C11, cy * face_mob_pc(w[2 * PL], w[3 * PL], hm));
+        link(C01, C11, cx * face_mob_pc(w[1], w[ld + 1], hm));
+        link(C10, C11, cy * face_mob_pc(w[ld], w[ld + 1], hm));
     }
 #pragma unroll
     for (int r = 0; r < n; r++) {
@@ -667,60 +678,111 @@ __device__ __forceinline__ void bot5_inverse(const T *w, T cx, T cy, int hm, int
     for (int r = 0; r < n; r++) inv[r * n + k] = sol[r];
 }
 
+// w of block (bi, bj) and around it, indices clamped into the level (a clamped
+// value only enters a face that is dropped), and its faces
 template <typename T>
-__device__ __forceinline__ void bot_preload(const BottomArgs<T> &A, BotShared<T, false> &s) {
-    // w of every depth: the depth and block of a thread are those of its work
-    // (threads 0..255 hold several depths).  Addresses are clamped into the
-    // level, so that every load is issued before the first is waited for.
-    T v[BOT_DEPTHS][4];
-    const int t = threadIdx.x;
+__device__ __forceinline__ void co5_from_w(const T *w, int ldw, int n1, int n2, int bi, int bj, T cx, T cy, int hm,
+                                           Co5<T> &k) {
+    const int i0 = 2 * bi, j0 = 2 * bj;
+    auto at = [&](int i, int j) -> T {
+        i = i < 0 ? 0 : (i > n1 - 1 ? n1 - 1 : i);
+        j = j < 0 ? 0 : (j > n2 - 1 ? n2 - 1 : j);
+        return w[(long)i * ldw + j];
+    };
+    const T c[4] = {at(i0, j0), at(i0, j0 + 1), at(i0 + 1, j0), at(i0 + 1, j0 + 1)};
+    const T wu[2] = {at(i0 - 1, j0), at(i0 - 1, j0 + 1)}, wd[2] = {at(i0 + 2, j0), at(i0 + 2, j0 + 1)};
+    const T wl[2] = {at(i0, j0 - 1), at(i0 + 1, j0 - 1)}, wr[2] = {at(i0, j0 + 2), at(i0 + 1, j0 + 2)};
+    make_co5(c, wu, wd, wl, wr, bi, bj, n1, n2, cx, cy, hm, k);
+}
+
+// Co5 as an array of BOT_CO values, and back
+template <typename T, class F>
+__device__ __forceinline__ void co5_each(Co5<T> &k, F &&f) {
 #pragma unroll
-    for (int d = 0; d < BOT_DEPTHS; d++) {
-        const int p = 5 - d;
-        const int l = d < A.d0 ? 0 : (d - A.d0 >= A.nl ? A.nl - 1 : d - A.d0);
-        const BotSize<T> L(A, l + A.d0);
-        const T *w = A.lev[l].w;
-        const int ld = A.lev[l].ldw;
-        const int i0 = min(2 * (t >> p), L.n1 - 1), i1 = min(i0 + 1, L.n1 - 1);
-        const int j0 = min(2 * (t & ((1 << p) - 1)), L.n2 - 1), j1 = min(j0 + 1, L.n2 - 1);
-        v[d][0] = w[i0 * ld + j0];
-        v[d][1] = w[i0 * ld + j1];
-        v[d][2] = w[i1 * ld + j0];
-        v[d][3] = w[i1 * ld + j1];
+    for (int q = 0; q < 2; q++) {
+        f(q, k.W[q]);
+        f(2 + q, k.E[q]);
+        f(4 + q, k.S[q]);
+        f(6 + q, k.N[q]);
+        f(8 + q, k.iE[q]);
+        f(10 + q, k.iN[q]);
     }
-    // the ring enters dropped faces only, but must be finite
-    for (int q = t; q < BotGeo::CELLS; q += blockDim.x) s.w[q] = T(1);
-    __syncthreads();
 #pragma unroll
-    for (int d = 0; d < BOT_DEPTHS; d++) {
+    for (int q = 0; q < 4; q++) f(12 + q, k.rc[q]);
+}
+
+// the coefficients of one depth (workgroup `d` of 6, 1024 threads), and the
+// coarsest level's solution operator (workgroup 5)
+template <typename T>
+__device__ __forceinline__ void bot5_setup_body(const BottomArgs<T> &A, int d, T *img, double *inv) {
+    const int t = threadIdx.x, dl = A.d0 + A.nl - 1;
+    if (d < BOT_DEPTHS - 1) {
         const int p = 5 - d;
-        if (d < A.d0 || t >= 1 << (2 * p)) continue;
-        const int o = BotGeo::origin(d) + ((t >> p) + 1) * BotGeo::LD + (t & ((1 << p) - 1)) + 1;
-#pragma unroll
-        for (int q = 0; q < 4; q++) s.w[q * BotGeo::PLANE + o] = v[d][q];
+        if (d < A.d0 || d >= dl || t >= 1 << (2 * p)) return;
+        const BotSize<T> L(A, d);
+        const int bi = t >> p, bj = t & ((1 << p) - 1);
+        const bool act = 2 * bi < L.n1 && 2 * bj < L.n2;
+        Co5<T> k;
+        if (act) {
+            const BotLev<T> &v = A.lev[d - A.d0];
+            co5_from_w(v.w, v.ldw, L.n1, L.n2, bi, bj, L.cx, L.cy, A.harmonic, k);
+        } else {
+            co5_each(k, [](int, T &v) { v = T(0); });
+        }
+        T *out = d == 0 ? img + t : img + BOT_CO * 1024 + bot_rhs_at(d) / 4 + t;
+        const int blocks = d == 0 ? 1024 : BOT_SMALL;
+        co5_each(k, [&](int q, T &v) { out[q * blocks] = v; });
+    } else {
+        const BotSize<T> L(A, dl);
+        const BotLev<T> &v = A.lev[A.nl - 1];
+        if (t >= L.n1 * L.n2) return;
+        // the hierarchy is coarsened until both sides are at most 2
+        if (L.n1 == 2 && L.n2 == 2) bot5_inverse<2, 2>(v.w, v.ldw, L.cx, L.cy, A.harmonic, t, inv);
+        else if (L.n1 == 2 && L.n2 == 1) bot5_inverse<2, 1>(v.w, v.ldw, L.cx, L.cy, A.harmonic, t, inv);
+        else if (L.n1 == 1 && L.n2 == 2) bot5_inverse<1, 2>(v.w, v.ldw, L.cx, L.cy, A.harmonic, t, inv);
+        else bot5_inverse<1, 1>(v.w, v.ldw, L.cx, L.cy, A.harmonic, t, inv);
     }
 }
-__device__ __forceinline__ void bot_preload(const BottomArgs<double> &A, BotShared<double, true> &s) {
+
+// what is read before the first barrier: the coefficients and the right-hand side
+// of the first level (k0: at depth 0, the others are in LDS), and what goes to LDS
+template <typename T>
+__device__ __forceinline__ void bot_preload(const BottomArgs<T> &A, BotShared<T, false> &s, int bi, int bj, bool act,
+                                            Co5<T> &k0) {
+    const int t = threadIdx.x, nt = blockDim.x;
+    if (act && A.d0 == 0) co5_each(k0, [&](int q, T &v) { v = A.img[q * 1024 + t]; });
+    constexpr int N = BOT_CO * BOT_SMALL * (int)sizeof(T) / 16;
+    static_assert(N * 16 == BOT_CO * BOT_SMALL * (int)sizeof(T), "copied 16 bytes at a time");
+    const double2 *src = reinterpret_cast<const double2 *>(A.img + BOT_CO * 1024);
+    double2 *dst = reinterpret_cast<double2 *>(s.co);
+    for (int base = t; base < N; base += 4 * nt) {
+        double2 v[4];
+#pragma unroll
+        for (int u = 0; u < 4; u++) v[u] = src[min(base + u * nt, N - 1)];
+#pragma unroll
+        for (int u = 0; u < 4; u++)
+            if (base + u * nt < N) dst[base + u * nt] = v[u];
+    }
+    if (t < 16) s.inv[t] = A.inv[t];
+}
+__device__ __forceinline__ void bot_preload(const BottomArgs<double> &A, BotShared<double, true> &s, int bi, int bj,
+                                            bool act, Co9<double> &k0) {
     if (threadIdx.x < 16) s.inv[threadIdx.x] = A.inv[threadIdx.x];
 }
 
-// the coefficients of block (bi, bj) of depth d (place o in the planes)
+// the coefficients of block (bi, bj) of depth d
 template <typename T>
-__device__ __forceinline__ void bot_coeffs(const BottomArgs<T> &A, const BotSize<T> &L, const BotShared<T, false> &s,
-                                           int d, int bi, int bj, int o, Co5<T> &k) {
-    using G = BotGeo;
-    T w[4];
-#pragma unroll
-    for (int q = 0; q < 4; q++) w[q] = s.w[q * G::PLANE + o];
-    const T wu[2] = {blk_nb<G, 0, 0, -1, 0>(w, s.w, o), blk_nb<G, 0, 1, -1, 0>(w, s.w, o)};
-    const T wd[2] = {blk_nb<G, 1, 0, 1, 0>(w, s.w, o), blk_nb<G, 1, 1, 1, 0>(w, s.w, o)};
-    const T wl[2] = {blk_nb<G, 0, 0, 0, -1>(w, s.w, o), blk_nb<G, 1, 0, 0, -1>(w, s.w, o)};
-    const T wr[2] = {blk_nb<G, 0, 1, 0, 1>(w, s.w, o), blk_nb<G, 1, 1, 0, 1>(w, s.w, o)};
-    make_co5(w, wu, wd, wl, wr, bi, bj, L.n1, L.n2, L.cx, L.cy, A.harmonic, k);
+__device__ __forceinline__ void bot_coeffs(const BottomArgs<T> &A, const BotShared<T, false> &s, int d, int bi, int bj,
+                                           const Co5<T> &k0, Co5<T> &k) {
+    if (d == 0) {
+        k = k0;
+        return;
+    }
+    const int at = bot_rhs_at(d) / 4 + (int)threadIdx.x;
+    co5_each(k, [&](int q, T &v) { v = s.co[q * BOT_SMALL + at]; });
 }
-__device__ __forceinline__ void bot_coeffs(const BottomArgs<double> &A, const BotSize<double> &L,
-                                           const BotShared<double, true> &s, int d, int bi, int bj, int o,
-                                           Co9<double> &k) {
+__device__ __forceinline__ void bot_coeffs(const BottomArgs<double> &A, const BotShared<double, true> &s, int d, int bi,
+                                           int bj, const Co9<double> &k0, Co9<double> &k) {
     load_co9(A.lev[d - A.d0].A, bi, bj, k);
 }
 template <typename T>
@@ -736,16 +798,26 @@ __device__ __forceinline__ void bot_diag(const BottomArgs<double> &A, const BotS
     load_diag9(A.lev[d - A.d0].A, bi, bj, c);
 }
 
+// the right-hand side of the bottom's first level
+template <typename T>
+__device__ __forceinline__ void bot_rhs0(const BottomArgs<T> &A, int bi, int bj, T (&b)[4]) {
+    const T *bp = A.b + (long)(2 * bi) * A.ldb + 2 * bj;
+    const bool v1 = 2 * bj + 1 < A.n2, w1 = 2 * bi + 1 < A.n1;
+    b[0] = bp[0];
+    b[1] = v1 ? bp[1] : T(0);
+    b[2] = w1 ? bp[A.ldb] : T(0);
+    b[3] = v1 && w1 ? bp[A.ldb + 1] : T(0);
+}
+// that of depth d: of the first level b0 (9-point: read again, its registers are
+// needed for the operator), of the others from LDS
 template <typename T, bool NINE>
-__device__ __forceinline__ void bot_rhs(const BottomArgs<T> &A, const BotSize<T> &L, const BotShared<T, NINE> &s, int d,
-                                        int bi, int bj, T (&b)[4]) {
-    if (d == A.d0) {
-        const T *bp = A.b + (long)(2 * bi) * A.ldb + 2 * bj;
-        const bool v1 = 2 * bj + 1 < L.n2, w1 = 2 * bi + 1 < L.n1;
-        b[0] = bp[0];
-        b[1] = v1 ? bp[1] : T(0);
-        b[2] = w1 ? bp[A.ldb] : T(0);
-        b[3] = v1 && w1 ? bp[A.ldb + 1] : T(0);
+__device__ __forceinline__ void bot_rhs(const BottomArgs<T> &A, const BotShared<T, NINE> &s, int d, int bi, int bj,
+                                        const T (&b0)[4], T (&b)[4]) {
+    if (NINE && d == A.d0) {
+        bot_rhs0(A, bi, bj, b);
+    } else if (d == A.d0) {
+#pragma unroll
+        for (int q = 0; q < 4; q++) b[q] = b0[q];
     } else {
         const int pp = 1 << (2 * (5 - d)), at = bot_rhs_at(d) + (int)threadIdx.x;
 #pragma unroll
@@ -759,9 +831,16 @@ __device__ __forceinline__ void mg_bottom_body(const BottomArgs<T> &A, BotShared
     using G = BotGeo;
     using GR = BotResGeo;
     const int t = threadIdx.x, dl = A.d0 + A.nl - 1;   // the coarsest level's depth
+    Co k0;
+    T b0[4] = {T(0), T(0), T(0), T(0)};
+    {
+        const int p = 5 - A.d0, bi = t >> p, bj = t & ((1 << p) - 1);
+        const bool act = t < 1 << (2 * p) && 2 * bi < A.n1 && 2 * bj < A.n2;
+        if (!NINE && act) bot_rhs0(A, bi, bj, b0);
+        bot_preload(A, s, bi, bj, act, k0);
+    }
     for (int q = t; q < BotShared<T, NINE>::CLEAR16; q += blockDim.x)
         reinterpret_cast<double2 *>(s.x)[q] = double2{0., 0.};
-    bot_preload(A, s);
     __syncthreads();
     // down: sweeps from a zero guess, residual, full weighting
     for (int d = A.d0; d < dl; d++) {
@@ -774,8 +853,8 @@ __device__ __forceinline__ void mg_bottom_body(const BottomArgs<T> &A, BotShared
         Co k;
         T b[4], x[4] = {T(0), T(0), T(0), T(0)}, r[4];
         if (act) {
-            bot_rhs(A, L, s, d, bi, bj, b);
-            bot_coeffs(A, L, s, d, bi, bj, o, k);
+            bot_rhs<T, NINE>(A, s, d, bi, bj, b0, b);
+            bot_coeffs(A, s, d, bi, bj, k0, k);
         }
         blk_sweeps<G, false>(k, b, x, s.x, o, act, A.ns, wg);
         if (act) {
@@ -798,19 +877,6 @@ __device__ __forceinline__ void mg_bottom_body(const BottomArgs<T> &A, BotShared
         blk_sync(wg);
     }
     const BotSize<T> Lb(A, dl);
-    if constexpr (!NINE) {
-        if (t >= 64 && t < 128) {
-            const int k = t - 64;
-            const T *w = s.w + G::origin(5) + G::LD + 1;
-            const T cx = Lb.cx, cy = Lb.cy;
-            if (k < Lb.n1 * Lb.n2) {   // the hierarchy is coarsened until both sides are at most 2
-                if (Lb.n1 == 2 && Lb.n2 == 2) bot5_inverse<2, 2>(w, cx, cy, A.harmonic, k, s.inv);
-                else if (Lb.n1 == 2 && Lb.n2 == 1) bot5_inverse<2, 1>(w, cx, cy, A.harmonic, k, s.inv);
-                else if (Lb.n1 == 1 && Lb.n2 == 2) bot5_inverse<1, 2>(w, cx, cy, A.harmonic, k, s.inv);
-                else bot5_inverse<1, 1>(w, cx, cy, A.harmonic, k, s.inv);
-            }
-        }
-    }
     __syncthreads();
     if (t < 64) {
         const int r = t >> 1, c = t & 1;   // cell (r, c) on lane 2 r + c
@@ -850,8 +916,8 @@ __device__ __forceinline__ void mg_bottom_body(const BottomArgs<T> &A, BotShared
             blk_prolong(e, x);
 #pragma unroll
             for (int q = 0; q < 4; q++) s.x[q * G::PLANE + o] = x[q];
-            bot_rhs(A, L, s, d, bi, bj, b);
-            bot_coeffs(A, L, s, d, bi, bj, o, k);
+            bot_rhs<T, NINE>(A, s, d, bi, bj, b0, b);
+            bot_coeffs(A, s, d, bi, bj, k0, k);
         }
         blk_sync(wg);
         blk_sweeps<G, true>(k, b, x, s.x, o, act, A.ns, wg);
@@ -902,18 +968,7 @@ __device__ __forceinline__ void leg5_inputs(const Leg5Args<T> &A, int bi, int bj
     b[1] = v1 ? bp[1] : T(0);
     b[2] = w1 ? bp[A.ld] : T(0);
     b[3] = v1 && w1 ? bp[A.ld + 1] : T(0);
-    // w of the block and around it, indices clamped into the level (a clamped
-    // value only enters a face that is dropped)
-    const int i0 = 2 * bi, j0 = 2 * bj;
-    auto at = [&](int i, int j) -> T {
-        i = i < 0 ? 0 : (i > A.n1 - 1 ? A.n1 - 1 : i);
-        j = j < 0 ? 0 : (j > A.n2 - 1 ? A.n2 - 1 : j);
-        return A.w[(long)i * A.ldw + j];
-    };
-    const T w[4] = {at(i0, j0), at(i0, j0 + 1), at(i0 + 1, j0), at(i0 + 1, j0 + 1)};
-    const T wu[2] = {at(i0 - 1, j0), at(i0 - 1, j0 + 1)}, wd[2] = {at(i0 + 2, j0), at(i0 + 2, j0 + 1)};
-    const T wl[2] = {at(i0, j0 - 1), at(i0 + 1, j0 - 1)}, wr[2] = {at(i0, j0 + 2), at(i0 + 1, j0 + 2)};
-    make_co5(w, wu, wd, wl, wr, bi, bj, A.n1, A.n2, T(A.cx), T(A.cy), A.harmonic, k);
+    co5_from_w(A.w, A.ldw, A.n1, A.n2, bi, bj, T(A.cx), T(A.cy), A.harmonic, k);
 }
 
 // tile `wg` of a down leg: sweeps from a zero guess, residual, full weighting
