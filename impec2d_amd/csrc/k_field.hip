@@ -549,7 +549,7 @@ __device__ __forceinline__ void tr_body(const G &gr_, double *__restrict__ c, co
     const int t = threadIdx.x;
     // the ordered sum of up to TR_ORDERED terms runs over LDS (a global load
     // per term, one after the other, took 250 us for the 2540 well cells of the
-    // 566^2 grid; 11 us so, the additions' own latency)
+    // 566^2 grid; 17 us so, the additions' own latency)
     __shared__ __attribute__((aligned(16))) double smd[TR_ORDERED];
     const bool ordered = nsrc <= TR_ORDERED;
     for (int k = t; k < nsrc; k += blockDim.x) {
