@@ -509,11 +509,13 @@ __device__ __forceinline__ T face_mob_pc(T wl, T wr, int harmonic) {
 
 // the faces of block (bi, bj) of an n1 x n2 level from its cells' w and the
 // eight cells around it: wu / wd the cells beyond the block in rows 2 bi - 1
-// and 2 bi + 2, wl / wr those in columns 2 bj - 1 and 2 bj + 2.  The sums wl + wr
-// of faces outside the level must be finite and not zero: those faces are
-// dropped by a zero factor, not by a branch around them (twelve short branches
-// cost four times the twelve reciprocals run together), and the averaging
-// procedure is chosen the same way: ch / s + cm s with one of the two zero.
+// and 2 bi + 2, wl / wr those in columns 2 bj - 1 and 2 bj + 2.  Faces outside the
+// level are dropped by a zero factor, not by a branch around them (twelve short
+// branches cost four times the twelve reciprocals run together): their cells' w
+// must be finite and, for the harmonic average, not zero.  The averaging
+// procedure is chosen the same way, ch / s + cm s with one of the two zero; for
+// the mean concentration the reciprocal is taken of 1, since the sum s of two
+// cells without permeability is zero there, and the face is too.
 template <typename T>
 __device__ __forceinline__ void make_co5(const T (&w)[4], const T (&wu)[2], const T (&wd)[2], const T (&wl)[2],
                                          const T (&wr)[2], int bi, int bj, int n1, int n2, T cx, T cy, int hm,
@@ -524,7 +526,7 @@ __device__ __forceinline__ void make_co5(const T (&w)[4], const T (&wu)[2], cons
     auto face = [&](T a, T b, T c, bool in) {
         const T f = in ? c : T(0), s = a + b;
         const T fh = hm ? T(2) * f : T(0), fm = hm ? T(0) : T(0.5) * f;
-        return fh * recip(s) + fm * s;
+        return fh * recip(hm ? s : T(1)) + fm * s;
     };
     k.W[0] = face(wu[0], w[0], cx, u);
     k.W[1] = face(wu[1], w[1], cx, u && c1);
