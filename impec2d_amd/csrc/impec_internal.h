@@ -77,10 +77,15 @@ enum { EST_DONE = 0, EST_ITER = 1, EST_CHECK = 2 };
 #ifndef IMPEC_STALL_ITS
 #define IMPEC_STALL_ITS 20
 #endif
-// ... or, once its norm is below the rounding floor that the solve before this
-// one met, in IMPEC_STALL_FLOOR_ITS: there the wait for 20 buys nothing (141^2
-// cells, eps 1e-14: the true residual is 2.1e-12 after 18 iterations and 2.1e-12
-// after 38).
+// In the consistent formulation the two are looked at earlier, after
+// IMPEC_STALL_FLOOR_ITS such iterations and without touching the iterate, and a
+// residual at the floor ends the solve: with a tolerance below it half the
+// iterations were the wait for the 20, in which p did not change by a bit
+// (141^2 cells, nu = 2/3, eps 1e-14: 38 -> 23 iterations; 283^2 35 -> 22; 566^2
+// 36 -> 21).  Not in the eliminated formulation, where the iterations after
+// that still bring the residual down by a third, nor with FP32 vectors, whose
+// corrections p does not hold.  A look costs one pass over p; solves that reach
+// their tolerance seldom stand still for 5 iterations.
 #ifndef IMPEC_STALL_FLOOR_ITS
 #define IMPEC_STALL_FLOOR_ITS 5
 #endif

@@ -822,6 +822,17 @@ __global__ void k_shift(CgArgs c, double *__restrict__ p, const double *__restri
     shift_body(HwGrid{}, c, p, S);
 }
 
+// out = what k_read_pin and k_shift would make of p, which stays as it is
+__global__ void k_shifted(CgArgs c, const double *__restrict__ p, double *__restrict__ out) {
+    const double sh = c.ppin - p[(long)(c.pin_i + c.B) * c.ldp + (c.pin_j + c.B)];
+    for (long id = (long)blockIdx.x * blockDim.x + threadIdx.x; id < c.n; id += (long)gridDim.x * blockDim.x) {
+        int i, j;
+        cg_cell(c, id, i, j);
+        const long o = (long)(i + c.B) * c.ldp + (j + c.B);
+        out[o] = (i == c.pin_i && j == c.pin_j) ? c.ppin : p[o] + sh;
+    }
+}
+
 // ||b - A x||^2 of the reference's pinned system
 template <bool DIAG, class G>
 __device__ __forceinline__ void true_residual_body(const G &gr_, LevArgs L, CgArgs c, const double *__restrict__ p, const double *__restrict__ q,
@@ -2941,7 +2952,6 @@ static int solve_cg(impec_ctx *ctx, int *its_out, double *relres_out) {
     int its = 0, status = IMPEC_OK;
     double relres = 0., rr = 0.;
     double floor_rel = 0., tol_eff = tol;   // the true residual's rounding floor, max(tol, floor)
-    const double floor_hint = ctx->stats.last_relres_floor;   // that of the solve before (0: none yet)
     double *dold = ctx->pd, *dnew = ctx->pz;
     float *dold32 = ctx->pd32, *dnew32 = ctx->pz32;
     double rr_ref = 0.;   // FP64 residual norm^2 at the FP32 recursion's last restart
@@ -2969,6 +2979,25 @@ static int solve_cg(impec_ctx *ctx, int *its_out, double *relres_out) {
             return st;
         }
         rr_ref = rr;
+        // true relative residual of x in the reference's pinned system, and its floor
+        auto pinned_residual = [&](const double *x, double &rel, double &flr) -> int {
+            int nparts = nb;
+            const TresArgs ta = tres_args(a0, c, x, ctx->q, ctx->part);
+            if (!DIAG && ta.nwave <= RED_BLOCKS) {   // the 5-point operator: the streamed pass
+                hipLaunchKernelGGL(k_true_rows, dim3(ta.gx), dim3(64 * SW_WAVES), 0, s, ta);
+                nparts = ta.nwave;
+            } else {
+                hipLaunchKernelGGL(k_true_residual<DIAG>, dim3(nb), dim3(256), 0, s, a0, c, x, ctx->q, ctx->part);
+            }
+            IMPEC_HIP_CHECK(ctx, hipGetLastError());
+            int e = finish_sum(ctx, nparts, 2, S_TT, pub_next(ctx));
+            if (!e) e = wait_scalars(ctx);
+            if (!e) {
+                rel = ctx->bnorm > 0 ? sqrt(ctx->h_scal[S_TT]) / ctx->bnorm : 0.;
+                flr = ctx->bnorm > 0 ? IMPEC_FLOOR_C * 0x1p-53 * sqrt(ctx->h_scal[S_FLOOR]) / ctx->bnorm : 0.;
+            }
+            return e;
+        };
         // p to the reference's pinned system (the shift, or the pinned value) and
         // that system's true relative residual
         auto finish_phase = [&]() -> int {
@@ -2978,23 +3007,19 @@ static int solve_cg(impec_ctx *ctx, int *its_out, double *relres_out) {
             } else {
                 hipLaunchKernelGGL(k_set_pin, dim3(1), dim3(1), 0, s, c, ctx->p);
             }
-            int nparts = nb;
-            const TresArgs ta = tres_args(a0, c, ctx->p, ctx->q, ctx->part);
-            if (!DIAG && ta.nwave <= RED_BLOCKS) {   // the 5-point operator: the streamed pass
-                hipLaunchKernelGGL(k_true_rows, dim3(ta.gx), dim3(64 * SW_WAVES), 0, s, ta);
-                nparts = ta.nwave;
-            } else {
-                hipLaunchKernelGGL(k_true_residual<DIAG>, dim3(nb), dim3(256), 0, s, a0, c, ctx->p, ctx->q,
-                                   ctx->part);
-            }
-            IMPEC_HIP_CHECK(ctx, hipGetLastError());
-            int e = finish_sum(ctx, nparts, 2, S_TT, pub_next(ctx));
-            if (!e) e = wait_scalars(ctx);
-            if (!e) {
-                relres = ctx->bnorm > 0 ? sqrt(ctx->h_scal[S_TT]) / ctx->bnorm : 0.;
-                floor_rel = ctx->bnorm > 0 ? IMPEC_FLOOR_C * 0x1p-53 * sqrt(ctx->h_scal[S_FLOOR]) / ctx->bnorm : 0.;
-                tol_eff = tol > floor_rel ? tol : floor_rel;
-            }
+            const int e = pinned_residual(ctx->p, relres, floor_rel);
+            if (!e) tol_eff = tol > floor_rel ? tol : floor_rel;
+            return e;
+        };
+        // whether finish_phase would find a residual at the floor (consistent phase);
+        // p, the recursion and tol_eff stay as they are.  t1 is the transport's,
+        // which is not under way.  floor_seen: the floor at the last look (-1: none)
+        double floor_seen = -1.;
+        auto at_floor_now = [&](bool &yes) -> int {
+            double rel = 0.;
+            hipLaunchKernelGGL(k_shifted, dim3(nb), dim3(256), 0, s, c, ctx->p, ctx->t1);
+            const int e = pinned_residual(ctx->t1, rel, floor_seen);
+            yes = !e && rel <= floor_seen;
             return e;
         };
         int since = 0, restarts = 0;
@@ -3046,8 +3071,14 @@ static int solve_cg(impec_ctx *ctx, int *its_out, double *relres_out) {
                 if (rr <= 0.25 * rr_mark) {
                     rr_mark = rr;
                     stall = 0;
-                } else if (++stall >= (rr <= floor_hint * floor_hint * bb ? IMPEC_STALL_FLOOR_ITS : IMPEC_STALL_ITS) &&
-                           rr == rr && !(rr <= tol * tol * bb)) {
+                } else if (++stall == IMPEC_STALL_FLOOR_ITS && c.shift && !ru && rr == rr &&
+                           !(rr <= tol * tol * bb) && (floor_seen < 0. || rr <= floor_seen * floor_seen * bb)) {
+                    if ((st = at_floor_now(at_floor))) return st;
+                    if (at_floor) {
+                        if ((st = finish_phase())) return st;
+                        break;
+                    }
+                } else if (stall >= IMPEC_STALL_ITS && rr == rr && !(rr <= tol * tol * bb)) {
                     // the pinned system's true residual and floor (p moves by a
                     // constant in the consistent phase, its pinned value is kept
                     // in the elimination phase: the recursion is unchanged)
