@@ -8,7 +8,8 @@
 // 4096^2 cells, interleaved by one thread, in 143 ms).  One thread copies into
 // fresh pages at 10-14 GB/s; the link takes 57 GB/s.  Reading c, p and the
 // velocity of 4096^2 cells took 226 ms, 24 steps and that output 606; with the
-// staging (and two multigrid steps) they take 397.
+// staging (and two multigrid steps) they take 397.  Where there is no pinned memory
+// to be had the pageable copies serve.
 #include "impec_device.h"
 #include <atomic>
 #include <mutex>
@@ -192,15 +193,39 @@ static int get_chunks(impec_ctx *ctx, const Stage &st, double *dst, const double
     return IMPEC_OK;
 }
 
+// the same without staging memory: pageable 2-D copies, the velocity's components
+// interleaved on the host
+static int get_plain(impec_ctx *ctx, double *dst, const double *a, const double *b, int ld, int rows, int cols) {
+    auto get2d = [&](double *to, const double *from) -> int {
+        IMPEC_HIP_CHECK(ctx, hipMemcpy2DAsync(to, sizeof(double) * cols, from, sizeof(double) * ld, sizeof(double) * cols,
+                                              rows, hipMemcpyDeviceToHost, ctx->stream));
+        IMPEC_HIP_CHECK(ctx, hipStreamSynchronize(ctx->stream));
+        return IMPEC_OK;
+    };
+    if (!b) return get2d(dst, a);
+    std::vector<double> u((size_t)rows * cols), v((size_t)rows * cols);
+    int e = get2d(u.data(), a);
+    if (!e) e = get2d(v.data(), b);
+    for (size_t k = 0; !e && k < u.size(); k++) {
+        dst[2 * k] = u[k];
+        dst[2 * k + 1] = v[k];
+    }
+    return e;
+}
+
 int get_field(impec_ctx *ctx, double *dst, const double *a, const double *b, int ld, int rows, int cols) {
     Stage st;
-    if (!stage_take(st)) return set_error(ctx, IMPEC_ENOMEM, "pinned staging memory");
+    const bool staged = stage_take(st);
     int e;
     try {
-        e = get_chunks(ctx, st, dst, a, b, ld, rows, cols, ctx->t2, (size_t)(ctx->N1 + 2 * ctx->B) * ctx->lds);
+        if (staged)
+            e = get_chunks(ctx, st, dst, a, b, ld, rows, cols, ctx->t2, (size_t)(ctx->N1 + 2 * ctx->B) * ctx->lds);
+        else
+            e = get_plain(ctx, dst, a, b, ld, rows, cols);
     } catch (const std::bad_alloc &) {
         e = set_error(ctx, IMPEC_ENOMEM, "host memory");
     }
+    if (!staged) return e;
     if (e) hipStreamSynchronize(ctx->stream);   // no copy into the stage is left in flight
     stage_give(st);
     return e;

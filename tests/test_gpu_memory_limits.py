@@ -1,0 +1,63 @@
+"""What happens at the end of memory.  A child process loads tests/host/alloc_limit.c
+before the library, so that allocations fail where the test wants them to: fields
+are read without pinned staging memory."""
+import os
+import subprocess
+import sys
+
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+HEAD = """
+import ctypes, sys, threading
+import numpy as np
+shim = ctypes.CDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL)
+shim.alloc_limit.argtypes = [ctypes.c_size_t, ctypes.c_size_t]
+shim.alloc_peak.restype = ctypes.c_size_t
+ANY = 2 ** 64 - 1
+from impec2d_amd import capi
+
+def fields(n1, n2, seed):
+    g = capi.Context(capi.default_params(N1=n1, N2=n2))
+    rng = np.random.default_rng(seed)
+    c, p, v = (rng.standard_normal(s) for s in (g.scalar_shape(), g.scalar_shape(), g.velocity_shape()))
+    g.set_concentration(c)
+    g.set_pressure(p)
+    g.set_velocity(v)
+    return g, c, p, v
+
+def check(g, c, p, v):
+    assert np.array_equal(g.get_concentration(), c)
+    assert np.array_equal(g.get_pressure(), p)
+    assert np.array_equal(g.get_velocity(), v)
+"""
+
+
+@pytest.fixture(scope="module")
+def shim(tmp_path_factory):
+    so = str(tmp_path_factory.mktemp("shim") / "alloc_limit.so")
+    src = os.path.join(ROOT, "tests", "host", "alloc_limit.c")
+    subprocess.check_call(["gcc", "-shared", "-fPIC", "-O1", "-Wall", src, "-o", so, "-ldl", "-lpthread"])
+    return so
+
+
+def _child(shim, body):
+    r = subprocess.run([sys.executable, "-c", HEAD + body, shim], cwd=ROOT, stdout=subprocess.PIPE,
+                       stderr=subprocess.STDOUT, timeout=100, text=True)
+    assert r.returncode == 0 and "done" in r.stdout, r.stdout
+
+
+def test_fields_are_read_without_pinned_memory(gpu_lib, shim):
+    _child(shim, """
+for n1, n2 in ((2, 2), (65, 63), (723, 721), (1021, 1025)):
+    shim.alloc_limit(ANY, 1 << 20)
+    g, c, p, v = fields(n1, n2, n1)
+    check(g, c, p, v)
+    shim.alloc_limit(ANY, ANY)   # memory again
+    check(g, c, p, v)
+    g.close()
+print("done")
+""")
