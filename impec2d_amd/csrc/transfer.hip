@@ -9,7 +9,7 @@
 // fresh pages at 10-14 GB/s; the link takes 57 GB/s.  Reading c, p and the
 // velocity of 4096^2 cells took 226 ms, 24 steps and that output 606; with the
 // staging (and two multigrid steps) they take 397.  Where there is no pinned memory
-// to be had the pageable copies serve.
+// to be had, or none free, the pageable copies serve.
 #include "impec_device.h"
 #include <atomic>
 #include <mutex>
@@ -42,24 +42,21 @@ __global__ void __launch_bounds__(256) k_pack(const double *__restrict__ a, cons
 namespace {
 
 constexpr size_t STAGE_BYTES = 8u << 20;   // one half of a stage
-constexpr int STAGES_KEPT = 2;             // idle stages kept while contexts exist
+constexpr int STAGES_MAX = 8;              // stages of the process (128 MiB)
 constexpr int COPY_THREADS = 8;
 constexpr size_t THREADS_FROM = 4u << 20;  // bytes from which several threads copy
 
 // Pinned staging memory, shared by all contexts of the process: a call takes a
-// stage for itself and gives it back; at most STAGES_KEPT stay allocated, and
-// none once the last context is gone.
+// stage for itself and gives it back.  Stages are allocated as calls overlap and
+// kept while contexts exist, since allocating 16 MiB of pinned memory takes longer
+// than most reads (a limit of two kept ones made twelve threads allocate 80 times
+// in 288 reads); a call that finds all STAGES_MAX taken goes without one.
 struct Stage {
     char *half[2];
 };
 std::mutex stage_lock;
-Stage stage_idle[STAGES_KEPT];
-int stage_nidle = 0, stage_users = 0;
-
-void stage_free(Stage &s) {
-    if (s.half[0]) hipHostFree(s.half[0]);
-    s.half[0] = s.half[1] = nullptr;
-}
+Stage stage_idle[STAGES_MAX];
+int stage_nidle = 0, stage_count = 0, stage_users = 0;
 
 bool stage_take(Stage &s) {
     {
@@ -68,25 +65,23 @@ bool stage_take(Stage &s) {
             s = stage_idle[--stage_nidle];
             return true;
         }
+        if (stage_count == STAGES_MAX) return false;
+        stage_count++;
     }
-    s.half[0] = s.half[1] = nullptr;
     if (hipHostMalloc((void **)&s.half[0], 2 * STAGE_BYTES, hipHostMallocPortable) != hipSuccess) {
         (void)hipGetLastError();
+        std::lock_guard<std::mutex> g(stage_lock);
+        stage_count--;
         return false;
     }
     s.half[1] = s.half[0] + STAGE_BYTES;
     return true;
 }
 
-void stage_give(Stage &s) {
-    {
-        std::lock_guard<std::mutex> g(stage_lock);
-        if (stage_users > 0 && stage_nidle < STAGES_KEPT) {
-            stage_idle[stage_nidle++] = s;
-            return;
-        }
-    }
-    stage_free(s);
+// a stage that comes back belongs to a call on a context, so stage_users > 0
+void stage_give(const Stage &s) {
+    std::lock_guard<std::mutex> g(stage_lock);
+    stage_idle[stage_nidle++] = s;
 }
 
 // Slices of consecutive chunks copied by `n` threads, the caller among them:
@@ -159,8 +154,11 @@ void transfer_attach() {
 
 void transfer_detach() {
     std::lock_guard<std::mutex> g(stage_lock);
-    if (--stage_users == 0)
-        while (stage_nidle > 0) stage_free(stage_idle[--stage_nidle]);
+    if (--stage_users > 0) return;
+    while (stage_nidle > 0) {
+        hipHostFree(stage_idle[--stage_nidle].half[0]);
+        stage_count--;
+    }
 }
 
 // rows x cols of the device array a (pitch ld), or of a and b interleaved, into

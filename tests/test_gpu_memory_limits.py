@@ -1,6 +1,7 @@
 """What happens at the end of memory.  A child process loads tests/host/alloc_limit.c
 before the library, so that allocations fail where the test wants them to: fields
-are read without pinned staging memory."""
+are read without pinned staging memory, and many readers at a time neither fail nor
+allocate staging memory again and again."""
 import os
 import subprocess
 import sys
@@ -59,5 +60,27 @@ for n1, n2 in ((2, 2), (65, 63), (723, 721), (1021, 1025)):
     shim.alloc_limit(ANY, ANY)   # memory again
     check(g, c, p, v)
     g.close()
+print("done")
+""")
+
+
+def test_many_readers_share_a_bounded_number_of_stages(gpu_lib, shim):
+    """Twelve threads with contexts of their own read eight times each; the staging
+    memory stays allocated while contexts exist, at most eight pieces of it, and what
+    finds none free is read without."""
+    _child(shim, """
+state = [fields(700 + 31 * k, 600 + 17 * k, k) for k in range(12)]
+failed = []
+def work(s):
+    try:
+        for _ in range(8):
+            check(*s)
+    except BaseException as e:
+        failed.append(repr(e))
+threads = [threading.Thread(target=work, args=(s,)) for s in state]
+for t in threads: t.start()
+for t in threads: t.join()
+assert not failed, failed
+assert 1 <= shim.alloc_host_calls() <= 8, shim.alloc_host_calls()
 print("done")
 """)
