@@ -1,15 +1,15 @@
 // transfer.hip -- device fields to the caller's pageable host arrays.
 //
 // The host layouts are compact (and the velocity interleaved), the device ones
-// padded: a kernel packs a chunk of the host layout into device scratch, one
-// copy brings it into pinned staging memory, and threads copy it on into the
-// caller's array while the next chunk is packed and copied into the other half.
-// A pageable 2-D copy moves 3.2 GB/s here (135 MB in 41 ms; the velocity of
-// 4096^2 cells, interleaved by one thread, in 143 ms).  One thread copies into
-// fresh pages at 10-14 GB/s; the link takes 57 GB/s.  Reading c, p and the
-// velocity of 4096^2 cells took 226 ms, 24 steps and that output 606; with the
-// staging (and two multigrid steps) they take 397.  Where there is no pinned memory
-// to be had, or none free, the pageable copies serve.
+// padded: a kernel packs a chunk of the host layout straight into pinned staging
+// memory, and threads copy it on into the caller's array while the next chunk is
+// packed into the other half.  Nothing of the context is written.  The link takes
+// 57 GB/s, one thread copies into fresh pages at 10-14; a pageable 2-D copy moves
+// 3.2 GB/s here (135 MB in 41 ms; the velocity of 4096^2 cells, interleaved by one
+// thread, in 143 ms).  c and v of 64^2 cells take 14 and 15 us, of 1024^2 0.31 and
+// 0.47 ms, of 4096^2 2.7 and 5.3 ms; packed into device memory and copied from
+// there 30 and 52 us, 0.39 and 0.56 ms, 3.0 and 5.7 ms.  Where there is no pinned
+// memory to be had, or none free, the pageable copies serve.
 #include "impec_device.h"
 #include <atomic>
 #include <mutex>
@@ -52,7 +52,7 @@ constexpr size_t THREADS_FROM = 4u << 20;  // bytes from which several threads c
 // than most reads (a limit of two kept ones made twelve threads allocate 80 times
 // in 288 reads); a call that finds all STAGES_MAX taken goes without one.
 struct Stage {
-    char *half[2];
+    double *half[2], *dev[2];   // on the host, and as the device sees them
 };
 std::mutex stage_lock;
 Stage stage_idle[STAGES_MAX];
@@ -68,13 +68,17 @@ bool stage_take(Stage &s) {
         if (stage_count == STAGES_MAX) return false;
         stage_count++;
     }
-    if (hipHostMalloc((void **)&s.half[0], 2 * STAGE_BYTES, hipHostMallocPortable) != hipSuccess) {
+    s.half[0] = nullptr;
+    if (hipHostMalloc((void **)&s.half[0], 2 * STAGE_BYTES, hipHostMallocPortable | hipHostMallocMapped) != hipSuccess ||
+        hipHostGetDevicePointer((void **)&s.dev[0], s.half[0], 0) != hipSuccess) {
         (void)hipGetLastError();
+        if (s.half[0]) hipHostFree(s.half[0]);
         std::lock_guard<std::mutex> g(stage_lock);
         stage_count--;
         return false;
     }
-    s.half[1] = s.half[0] + STAGE_BYTES;
+    s.half[1] = s.half[0] + STAGE_BYTES / sizeof(double);
+    s.dev[1] = s.dev[0] + STAGE_BYTES / sizeof(double);
     return true;
 }
 
@@ -161,32 +165,30 @@ void transfer_detach() {
     }
 }
 
-// rows x cols of the device array a (pitch ld), or of a and b interleaved, into
-// dst; scratch: a device array of scratch_n doubles
+// rows x cols of the device array a (pitch ld), or of a and b interleaved, into dst
 static int get_chunks(impec_ctx *ctx, const Stage &st, double *dst, const double *a, const double *b, int ld, int rows,
-                      int cols, double *scratch, size_t scratch_n) {
+                      int cols) {
     const size_t total = (size_t)rows * cols * (b ? 2 : 1);
-    size_t per = STAGE_BYTES / sizeof(double);
-    if (per > scratch_n) per = scratch_n;
-    const size_t chunks = (total + per - 1) / per;
-    Copiers pool(copy_threads(total * sizeof(double)));
+    const size_t per = STAGE_BYTES / sizeof(double), chunks = (total + per - 1) / per;
     auto queue = [&](size_t c) -> int {
         const size_t at = c * per, n = per < total - at ? per : total - at;
         hipLaunchKernelGGL(k_pack, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, ctx->stream, a, b, ld,
-                           (unsigned long long)cols, (unsigned long long)at, (unsigned long long)n, scratch);
+                           (unsigned long long)cols, (unsigned long long)at, (unsigned long long)n, st.dev[c & 1]);
         IMPEC_HIP_CHECK(ctx, hipGetLastError());
-        IMPEC_HIP_CHECK(ctx, hipMemcpyAsync(st.half[c & 1], scratch, n * sizeof(double), hipMemcpyDeviceToHost,
-                                            ctx->stream));
         IMPEC_HIP_CHECK(ctx, hipEventRecord(ctx->ev_get[c & 1], ctx->stream));
         return IMPEC_OK;
     };
+    const int nthreads = copy_threads(total * sizeof(double));
+    // the copying threads look for work in turn: not before the stream has come to it
+    if (nthreads > 1) IMPEC_HIP_CHECK(ctx, hipStreamSynchronize(ctx->stream));
     if (int e = queue(0)) return e;
+    Copiers pool(nthreads);
     for (size_t c = 0; c < chunks; c++) {
         if (c + 1 < chunks)   // its half was emptied in the previous round
             if (int e = queue(c + 1)) return e;
         IMPEC_HIP_CHECK(ctx, hipEventSynchronize(ctx->ev_get[c & 1]));
         const size_t at = c * per, n = per < total - at ? per : total - at;
-        pool.copy((char *)(dst + at), st.half[c & 1], n * sizeof(double));
+        pool.copy((char *)(dst + at), (const char *)st.half[c & 1], n * sizeof(double));
     }
     return IMPEC_OK;
 }
@@ -217,7 +219,7 @@ int get_field(impec_ctx *ctx, double *dst, const double *a, const double *b, int
     int e;
     try {
         if (staged)
-            e = get_chunks(ctx, st, dst, a, b, ld, rows, cols, ctx->t2, (size_t)(ctx->N1 + 2 * ctx->B) * ctx->lds);
+            e = get_chunks(ctx, st, dst, a, b, ld, rows, cols);
         else
             e = get_plain(ctx, dst, a, b, ld, rows, cols);
     } catch (const std::bad_alloc &) {
