@@ -50,8 +50,18 @@ void prof_end(impec_ctx *ctx, const char *name) {
 
 static int round_up(int x, int m) { return (x + m - 1) / m * m; }
 
+hipError_t ctx_malloc_bytes(impec_ctx *ctx, void **p, size_t bytes) {
+    hipError_t e = hipMalloc(p, bytes);
+    if (e == hipSuccess) return e;
+    (void)hipGetLastError();
+    hipStreamSynchronize(ctx->stream);   // a solve that reads the planes may be under way
+    if (op9_free(ctx)) e = hipMalloc(p, bytes);
+    if (e != hipSuccess) (void)hipGetLastError();
+    return e;
+}
+
 static int dalloc(impec_ctx *ctx, double **p, size_t n) {
-    if (hipMalloc((void **)p, n * sizeof(double)) != hipSuccess) {
+    if (ctx_malloc(ctx, p, n * sizeof(double)) != hipSuccess) {
         *p = nullptr;
         return set_error(ctx, IMPEC_ENOMEM, "device allocation of %zu doubles failed", n);
     }
@@ -70,7 +80,7 @@ static int ensure_cn(impec_ctx *ctx) {
                      &ctx->cn_r2, &ctx->cn_y, &ctx->cn_z};
     for (int k = 0; k < 8; k++)
         if ((st = dalloc(ctx, v[k], n))) return st;
-    if (hipMalloc((void **)&ctx->cn_dg, n * sizeof(float)) != hipSuccess) {
+    if (ctx_malloc(ctx, &ctx->cn_dg, n * sizeof(float)) != hipSuccess) {
         ctx->cn_dg = nullptr;
         return set_error(ctx, IMPEC_ENOMEM, "device allocation of %zu floats failed", n);
     }
@@ -240,6 +250,7 @@ int impec::ctx_create(const impec_params *P, hipStream_t ext, impec_ctx **out) {
         if (!st) st = dalloc(ctx, &ctx->p_old, ns);
     }
     if (!st && P->diffusion) st = ensure_cn(ctx);
+    if (!st) op9_alloc(ctx);
     if (!st) update_symmetry(ctx);
     if (!st && hipDeviceSynchronize() != hipSuccess) st = set_error(ctx, IMPEC_EHIP, "initial synchronisation");
     if (st) {
@@ -351,9 +362,9 @@ int impec_set_source(impec_ctx *ctx, const double *q) {
     ctx->src_idx = nullptr; ctx->src_q = nullptr; ctx->tr_md = nullptr;
     ctx->nsrc = (int)idx.size();
     if (ctx->nsrc) {
-        IMPEC_HIP_CHECK(ctx, hipMalloc(&ctx->src_idx, sizeof(int) * ctx->nsrc));
-        IMPEC_HIP_CHECK(ctx, hipMalloc(&ctx->src_q, sizeof(double) * ctx->nsrc));
-        IMPEC_HIP_CHECK(ctx, hipMalloc(&ctx->tr_md, sizeof(double) * ctx->nsrc));
+        IMPEC_HIP_CHECK(ctx, ctx_malloc(ctx, &ctx->src_idx, sizeof(int) * ctx->nsrc));
+        IMPEC_HIP_CHECK(ctx, ctx_malloc(ctx, &ctx->src_q, sizeof(double) * ctx->nsrc));
+        IMPEC_HIP_CHECK(ctx, ctx_malloc(ctx, &ctx->tr_md, sizeof(double) * ctx->nsrc));
         IMPEC_HIP_CHECK(ctx, hipMemcpyAsync(ctx->src_idx, idx.data(), sizeof(int) * ctx->nsrc, hipMemcpyHostToDevice,
                                             ctx->stream));
         IMPEC_HIP_CHECK(ctx, hipMemcpyAsync(ctx->src_q, qv.data(), sizeof(double) * ctx->nsrc, hipMemcpyHostToDevice,
@@ -443,7 +454,7 @@ int impec_intercell_flux(impec_ctx *ctx, int dir, double dt, double *F) {
     const size_t n = dir == 0 ? (size_t)(ctx->N1 + 1) * (ctx->N2 + 2 * ctx->B)
                               : (size_t)(ctx->N1 + 2 * ctx->B) * (ctx->N2 + 1);
     double *d = nullptr;
-    IMPEC_HIP_CHECK(ctx, hipMalloc(&d, n * sizeof(double)));
+    IMPEC_HIP_CHECK(ctx, ctx_malloc(ctx, &d, n * sizeof(double)));
     int st = intercell_flux(ctx, dir, dt, d);
     hipError_t e = hipSuccess;
     if (!st) e = hipMemcpyAsync(F, d, n * sizeof(double), hipMemcpyDeviceToHost, ctx->stream);

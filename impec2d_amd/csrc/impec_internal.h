@@ -305,6 +305,12 @@ inline size_t sidx(const impec_ctx *ctx, int i, int j) {
     return (size_t)(i + ctx->B) * ctx->lds + (j + ctx->B);
 }
 
+// device memory of a context (capi.hip): hipMalloc, and once more without the
+// planes of the 9-point cycle where that fails
+hipError_t ctx_malloc_bytes(impec_ctx *ctx, void **p, size_t bytes);
+template <typename T>
+inline hipError_t ctx_malloc(impec_ctx *ctx, T **p, size_t bytes) { return ctx_malloc_bytes(ctx, (void **)p, bytes); }
+
 // ---- fields to the host (transfer.hip) ----
 // the host layout (rows x cols, compact) of device array a with pitch ld, or of
 // a and b interleaved (b not null); waits for the stream
@@ -350,6 +356,8 @@ int launch_minmax(impec_ctx *ctx, double *cmax, double *cmin);
 
 // ---- pressure (k_pressure.hip) ----
 int pressure_setup_levels(impec_ctx *ctx);
+void op9_alloc(impec_ctx *ctx);   // the optional planes of the 9-point cycle
+bool op9_free(impec_ctx *ctx);    // whether there were any
 void pressure_free_levels(impec_ctx *ctx);
 int pressure_solve(impec_ctx *ctx, int *its, double *relres);
 int pressure_operator_dump(impec_ctx *ctx, double *A9_host);

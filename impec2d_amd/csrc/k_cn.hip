@@ -1211,7 +1211,7 @@ int cn_operator_dump(impec_ctx *ctx, double dt, double *A9_host, double *rhs_hos
     int st = tensors_and_rhs(ctx, k);
     if (st) return st;
     double *dA = nullptr;
-    IMPEC_HIP_CHECK(ctx, hipMalloc(&dA, sizeof(double) * 9 * n));
+    IMPEC_HIP_CHECK(ctx, ctx_malloc(ctx, &dA, sizeof(double) * 9 * n));
     dim3 blk(64, 4), gc((ctx->N2 + 63) / 64, (ctx->N1 + 3) / 4);
     hipLaunchKernelGGL(k_cn_dump, gc, blk, 0, ctx->stream, k, ctx->u, ctx->v, dA);
     hipError_t e = hipGetLastError();

@@ -931,9 +931,6 @@ static LevArgs lev_args(const impec_ctx *ctx, int l) {
 
 static int round_up(int x, int m) { return (x + m - 1) / m * m; }
 
-static bool blocks9_ok(const impec_ctx *ctx);
-static bool op9_alloc(impec_ctx *ctx);
-
 int pressure_setup_levels(impec_ctx *ctx) {
     int n1 = ctx->N1, n2 = ctx->N2;
     double dx = ctx->dx, dy = ctx->dy;
@@ -970,26 +967,38 @@ int pressure_setup_levels(impec_ctx *ctx) {
         if (hipMalloc(vecs[k], bytes0) != hipSuccess) return set_error(ctx, IMPEC_ENOMEM, "CG vector allocation failed");
         hipMemset(*vecs[k], 0, bytes0);
     }
-    if (ctx->P.nu != 1. && blocks9_ok(ctx)) op9_alloc(ctx);
-    if (hipMalloc(&ctx->bot_img, bot_img_bytes<double>()) != hipSuccess)
-        return set_error(ctx, IMPEC_ENOMEM, "multigrid bottom allocation failed");
-    hipMemset(ctx->bot_img, 0, bot_img_bytes<double>());
+    if (ctx->P.nu == 1.) {   // the 5-point bottom's coefficients
+        if (hipMalloc(&ctx->bot_img, bot_img_bytes<double>()) != hipSuccess)
+            return set_error(ctx, IMPEC_ENOMEM, "multigrid bottom allocation failed");
+        hipMemset(ctx->bot_img, 0, bot_img_bytes<double>());
+    }
     return IMPEC_OK;
 }
 
+bool op9_free(impec_ctx *ctx) {
+    bool any = false;
+    for (int l = 0; l < MAX_LEVELS; l++)
+        if (ctx->lev[l].a9) {
+            hipFree(ctx->lev[l].a9);
+            ctx->lev[l].a9 = nullptr;
+            any = true;
+        }
+    if (ctx->op9_inv) hipFree(ctx->op9_inv);
+    ctx->op9_inv = nullptr;
+    return any;
+}
+
 void pressure_free_levels(impec_ctx *ctx) {
+    op9_free(ctx);
     for (int l = 0; l < ctx->nlev; l++) {
         Level &L = ctx->lev[l];
         hipFree(L.x); hipFree(L.b); hipFree(L.r);
         hipFree(L.wf); hipFree(L.wf2); hipFree(L.xf); hipFree(L.bf); hipFree(L.rf);
-        if (L.a9) hipFree(L.a9);
         if (L.w) hipFree(L.w);
     }
     ctx->nlev = 0;
     hipFree(ctx->pr); hipFree(ctx->pz); hipFree(ctx->pd); hipFree(ctx->pq);
     hipFree(ctx->fx); hipFree(ctx->fy);
-    if (ctx->op9_inv) hipFree(ctx->op9_inv);
-    ctx->op9_inv = nullptr;
     if (ctx->bot_img) hipFree(ctx->bot_img);
     if (ctx->bot_img32) hipFree(ctx->bot_img32);
     ctx->bot_img = ctx->bot_img32 = nullptr;
@@ -2441,9 +2450,12 @@ static bool blocks9_ok(const impec_ctx *ctx) {
     return ti * tj * 2 <= RED_BLOCKS;
 }
 
-// the planes of every level's assembled operator; false when the device has
-// no room for them (the one-kernel-per-pass cycle then runs)
-static bool op9_alloc(impec_ctx *ctx) {
+// The planes of every level's assembled operator: 107 B per cell that the solve
+// can do without, as the one-kernel-per-pass cycle then runs.  So they are
+// allocated when the context has all that it needs, may fail, and make room when
+// a later allocation of the context finds none (op9_free, ctx_malloc).
+void op9_alloc(impec_ctx *ctx) {
+    if (ctx->P.nu == 1. || !blocks9_ok(ctx)) return;
     bool ok = true;
     for (int l = 0; ok && l < ctx->nlev; l++) {
         Level &L = ctx->lev[l];
@@ -2455,15 +2467,8 @@ static bool op9_alloc(impec_ctx *ctx) {
     ok = ok && hipMalloc(&ctx->op9_inv, sizeof(double) * 16) == hipSuccess;
     if (!ok) {
         (void)hipGetLastError();
-        for (int l = 0; l < ctx->nlev; l++)
-            if (ctx->lev[l].a9) {
-                hipFree(ctx->lev[l].a9);
-                ctx->lev[l].a9 = nullptr;
-            }
-        if (ctx->op9_inv) hipFree(ctx->op9_inv);
-        ctx->op9_inv = nullptr;
+        op9_free(ctx);
     }
-    return ok;
 }
 
 static int op9_assemble(impec_ctx *ctx) {
@@ -3203,7 +3208,7 @@ int pressure_operator_dump(impec_ctx *ctx, double *A9_host) {
     LevArgs a0 = lev_args(ctx, 0);
     const size_t bytes = sizeof(double) * 9 * (size_t)ctx->N1 * ctx->N2;
     double *dA = nullptr;
-    IMPEC_HIP_CHECK(ctx, hipMalloc(&dA, bytes));
+    IMPEC_HIP_CHECK(ctx, ctx_malloc(ctx, &dA, bytes));
     dim3 blk(64, 4);
     const double dpin = ctx->kappa / ctx->dA;
     if (ctx->P.nu != 1.)

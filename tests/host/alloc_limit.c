@@ -10,7 +10,7 @@ enum { N_MAX = 4096, OUT_OF_MEMORY = 2 /* hipErrorOutOfMemory */ };
 
 static pthread_mutex_t lock = PTHREAD_MUTEX_INITIALIZER;
 static struct { void *p; size_t n; } blocks[N_MAX];
-static size_t live, peak, limit = (size_t)-1, host_limit = (size_t)-1;
+static size_t live, limit = (size_t)-1, host_limit = (size_t)-1;
 static int host_calls;
 
 void alloc_limit(size_t device_bytes, size_t host_block_bytes) {
@@ -19,7 +19,7 @@ void alloc_limit(size_t device_bytes, size_t host_block_bytes) {
     host_limit = host_block_bytes;
     pthread_mutex_unlock(&lock);
 }
-size_t alloc_peak(void) { return peak; }
+size_t alloc_live(void) { return live; }
 /* successful host allocations of at least 1 MiB */
 int alloc_host_calls(void) { return host_calls; }
 
@@ -48,7 +48,6 @@ int hipMalloc(void **p, size_t n) {
                 break;
             }
         live += n;
-        if (live > peak) peak = live;
     }
     pthread_mutex_unlock(&lock);
     return e;
