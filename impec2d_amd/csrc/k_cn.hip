@@ -81,21 +81,26 @@ __device__ __forceinline__ void yface_tensor(const CnConst &k, double ub, double
     d22 = x22;
 }
 
-// The two tensors with phi alpha / |u| formed from a reciprocal square root (the
-// hardware estimate and two Newton steps, y' = y + y (1/2 - (q/2) y^2), to about
-// an ulp) in place of a square root and two divisions: for the solver's own
-// operator applications, the s- and p-launches, whose rounding the true
-// residual with the exact tensors (CN_R, CN_RX) checks before a solve ends.  Those
+// The two tensors with phi alpha / |u| formed from a reciprocal square root in
+// place of a square root and two divisions, for the solver's own operator
+// applications, the s- and p-launches, whose rounding the true residual with the
+// exact tensors (CN_R, CN_RX) checks before a solve ends: the hardware estimate and
+// two Newton steps y' = y + y (1/2 - (q/2) y^2), the second with the rounding of
+// (q/2) y taken back.  Errors against 128 bits over 4e6 velocities of 2^-40 to 2^10
+// at alpha 1e-3 / 1e-4, d_m 1e-5, in units of 2^-53, r.m.s. and largest: d11 0.59
+// and 4.3 (with root and divisions 0.61 and 4.5), d12 0.93 and 4.0 (0.93 and 4.2);
+// without d_m, with equal alphas and over 2^-440 to 2^440 likewise.  Those
 // launches are limited by instruction issue as much as by bytes: at 4096^2 the
-// s-launch takes 168.5 us against 184.8 and the p-launch 295 against 304, at
-// 1024^2 20.5 against 25.7 and 28.6 against 33.2; the true residuals reached are
-// the same.  Outside the range where the steps neither overflow nor lose bits, and for
+// s-launch takes 170 us against 184.8 and the p-launch 296 against 304, at 1024^2
+// 20.8 against 25.7 and 28.7 against 33.2; the true residuals reached are the
+// same.  Outside the range where the steps neither overflow nor lose bits, and for
 // speed zero, the exact ones.
 __device__ __forceinline__ bool rsqrt_fast(double q, double &y) {
     const double h = 0.5 * q;
     y = __builtin_amdgcn_rsq(q);
     y = fma(y, fma(-(h * y), y, 0.5), y);
-    y = fma(y, fma(-(h * y), y, 0.5), y);
+    const double hy = h * y;
+    y = fma(y, fma(-fma(h, y, -hy), y, fma(-hy, y, 0.5)), y);
     return q >= 0x1p-900 && q <= 0x1p+900;
 }
 __device__ __forceinline__ void xface_tensor_fast(const CnConst &k, double uu, double vb, double &d11, double &d12) {
@@ -106,7 +111,7 @@ __device__ __forceinline__ void xface_tensor_fast(const CnConst &k, double uu, d
         return;
     }
     const double fl = k.phal * y, ft = k.phat * y;
-    d11 = fma(fl, u2, fma(ft, v2, k.phdm));
+    d11 = fma(fl, u2, ft * v2) + k.phdm;
     d12 = (fl - ft) * (uu * vb);
 }
 __device__ __forceinline__ void yface_tensor_fast(const CnConst &k, double ub, double vv, double &d22, double &d21) {

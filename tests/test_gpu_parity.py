@@ -216,6 +216,35 @@ def test_parabolic_solve_ragged_strips(gpu_lib, n1, n2, cn_guess):
     assert rel_err(cg.reshape(-1), x) < 1e-12
 
 
+@pytest.mark.parametrize("low,high,still", [(1.0, 1.0, True), (1e-150, 1e-150, True), (1e140, 1e140, False),
+                                            (1e-160, 1.0, False), (1e-136, 1e-130, False)])
+def test_parabolic_solve_over_the_range_of_speeds(gpu_lib, low, high, still):
+    """The solver's own tensors come from a reciprocal square root where |u|^2 lies
+    in 2^-900 .. 2^900 (1e-271 .. 8e270) and from the exact ones elsewhere and at
+    rest: speeds within, below and above that range, on both sides of its lower end
+    in one wave, and with a region at rest.  The time step and d_m go with the speed, so the
+    system is as well conditioned as the one above, and the bound is the same."""
+    from oracle import pyoracle as po
+    n1, n2 = 21, 63
+    p = params(N1=n1, N2=n2, diffusion=1, alpha_abs=1, alpha_l=0.02, alpha_t=0.005, d_m=1e-3 * high, para_eps=1e-14)
+    _say("parabolic solve speeds", low, high, still)
+    o, g = pair(p)
+    c = smooth_c(o, seed=31)
+    rng = np.random.default_rng(32)
+    v = (rng.standard_normal(o.velocity().shape) + 0.5) * np.where(np.arange(o.velocity().shape[1]) % 5 < 2, low, high)[:, None]
+    if still:
+        v[8:16, 20:45] = 0.0
+    o.fill_velocity(v)
+    g.set_concentration(c)
+    g.set_velocity(v)
+    dt = 3e-3 / high
+    its = g.dispersion_cn(dt)
+    x = po.dense_solve9(o.N1, o.N2, o.parabolic_matrix(v, dt), o.parabolic_rhs(c, v, dt))
+    cg = o.interior(g.get_concentration())
+    assert its > 0
+    assert rel_err(cg.reshape(-1), x) < 1e-12
+
+
 @pytest.mark.parametrize("kw", [dict(nu=1.0), dict(nu=2 / 3.0), dict(nu=2 / 3.0, stype=0, x_ub=2 ** 0.5,
                                                                       y_ub=2 ** 0.5),
                                 dict(nu=2 / 3.0, N1=24, N2=12), dict(nu=1.0, avgproc=1)])
