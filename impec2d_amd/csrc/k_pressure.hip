@@ -3030,6 +3030,7 @@ static int solve_cg(impec_ctx *ctx, int *its_out, double *relres_out) {
         int since = 0, restarts = 0;
         double rr_check = -1.;   // true residual norm^2 at the previous restart (-1: none yet)
         bool finished = false, at_floor = false;
+        bool with_constant = true;
         for (;;) {
             bool broke = false;
             double rr_mark = rr;   // the recursive residual when it last halved
@@ -3134,7 +3135,23 @@ static int solve_cg(impec_ctx *ctx, int *its_out, double *relres_out) {
             // restart while each restart at least halves the true residual
             // (up to IMPEC_MAX_RESTARTS), and at least 3 times
             const bool progress = rr_before < 0. || rr <= 0.25 * rr_before;
-            if (rr <= tol_eff * tol_eff * bb || restarts >= IMPEC_MAX_RESTARTS || (restarts >= 3 && !progress)) break;
+            if (rr <= tol_eff * tol_eff * bb) break;
+            if (restarts >= IMPEC_MAX_RESTARTS || (restarts >= 3 && !progress)) {
+                // spent.  With permeabilities over many decades the preconditioner's
+                // constant (pin_shift) overshoots, and rounding leaves the residual
+                // just above a tolerance near the floor: once more without it
+                if ((st = finish_phase())) return st;
+                if (relres <= tol_eff || !with_constant) {
+                    finished = true;
+                    break;
+                }
+                with_constant = false;
+                hipLaunchKernelGGL(k_fill_zero, dim3(1), dim3(1), 0, s, ctx->scal + S_PINSUM, 1l);
+                IMPEC_HIP_CHECK(ctx, hipGetLastError());
+                restarts_all += restarts;
+                restarts = -1;
+                rr_check = -1.;
+            }
             restarts++;
             since = 0;
         }

@@ -85,3 +85,20 @@ def test_eliminated_formulation_needs_no_search_for_the_constant(gpu_lib, n1, n2
         g.close()
     assert max(its) <= 20 and abs(its[0] - its[1]) <= 1, its
     assert rel_err(ps[0], ps[1]) < 1e-8
+
+
+@pytest.mark.parametrize("n1,n2,nu,seed", [(119, 125, 1 / 3, 171), (107, 120, 2 / 3, 199)])
+def test_eliminated_formulation_over_many_decades_of_permeability(gpu_lib, n1, n2, nu, seed):
+    """Anisotropic white-noise permeability of sigma 4 (over ten decades), with a
+    tolerance below the rounding floor: the preconditioner's constant, which
+    overshoots there, must not keep a solve from the floor that it reaches with the
+    V-cycle alone (0.92 and 0.27 of it; 1.2 times it with the constant throughout)."""
+    p = params(N1=n1, N2=n2, nu=nu, x_ub=n1 / n2, avgproc=1, mu_res=10.0, mu_inj=1.0, eps=1e-14, max_iter=3000)
+    rng = np.random.default_rng(seed)
+    K11, K22 = (np.exp(4.0 * rng.standard_normal((n1 + 4, n2 + 4))) for _ in range(2))
+    o, g = pair(p, K11, K22)
+    g.set_source(o.source())
+    g.set_concentration(smooth_c(o))
+    _, rr = g.pressure_solve()
+    assert rr <= g.stats().last_relres_floor
+    g.close()
