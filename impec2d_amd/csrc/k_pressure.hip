@@ -686,7 +686,9 @@ __global__ void k_sum(CgArgs c, const double *__restrict__ x0, double *__restric
 // a constant added to the V-cycle's output: v.A v = -sum of the neighbours'
 // coefficients towards the pinned cell (S_PINSUM, k_pin_sum), v.r = sum r.
 // Iterations to 1e-10 at nu = 2/3: 100 x 50 cells 28 -> 19, 300 x 290 30 -> 18,
-// 500 x 260 35 -> 21; nu = 0, 100 x 50: 97 -> 62.
+// 500 x 260 35 -> 21; nu = 0, 100 x 50: 97 -> 62.  Where v.A v is tiny beside the
+// other couplings the constant overshoots on the way, and its rounding stays in
+// the residual: solve_cg's last restarts go without it.
 __device__ __forceinline__ double pin_shift(int shift, const double *__restrict__ S) {
     return shift ? 0. : S[S_RSUM] * S[S_PINSUM];
 }
@@ -2182,11 +2184,11 @@ __global__ void k_cg_update2(CgArgs c, double *__restrict__ p, const double *__r
 #endif
 // rows per chunk of the streaming legs: about IMPEC_MG_WAVES wavefronts on large
 // levels, short chunks on small ones; even, since the march starts on an
-// even row.  The small levels' legs are a latency chain whose length is the
-// chunk plus the halo rows: on levels of at most IMPEC_MG_SMALL_ROWS rows
-// chunks of 2 rows make the step 0.4% faster than 4; on larger levels the
-// halo work of 2-row chunks costs more than it saves (512^2: 30 us per
-// V-cycle against 26), and they keep 4
+// even row.  The legs of a small grid's finest level (its coarser ones are tiles,
+// tile_level) are a latency chain whose length is the chunk plus the halo rows: on
+// levels of at most IMPEC_MG_SMALL_ROWS rows chunks of 2 rows made the step 0.4%
+// faster than 4; on larger levels the halo work of 2-row chunks costs more than
+// it saves (512^2: 30 us per V-cycle against 26), and they keep 4
 #ifndef IMPEC_MG_MINROWS
 #define IMPEC_MG_MINROWS 2
 #endif
@@ -2222,8 +2224,8 @@ template <> struct LevelArrays<float> {
     static float *r(const Level &L) { return L.rf; }
 };
 
-// red-black pairs per leg of the streaming legs: 2 for mg_pre = mg_post = 2,
-// else 1 (the single-workgroup bottom of the cycle always runs one pair)
+// red-black pairs per leg, on every level and in the bottom: 2 for mg_pre =
+// mg_post = 2, else 1
 static int mg_ns(const impec_ctx *ctx) { return ctx->P.mg_pre == 2 && ctx->P.mg_post == 2 ? 2 : 1; }
 
 template <typename T>
@@ -2713,8 +2715,10 @@ static DirMvArgs<T> dir_mv_args(impec_ctx *ctx, const LevArgs &a0, const CgArgs 
 // three iterations below: dir(fold, part) and upd(fold, part) launch the two
 // passes (fold.n > 0: they form the preceding sums themselves).  Folding saves
 // two launches of one workgroup (4 to 6 us each).  Every workgroup reads the
-// partials for it, so it is done while partials x workgroups stay below
-// IMPEC_FOLD_READS (grids up to about 600^2).
+// partials for it, so it is done while partials x workgroups stay within
+// IMPEC_FOLD_READS: up to 576^2 with the 5-point operator (720 partials of the
+// direction pass in 1296 workgroups), up to 512^2 with the 9-point one (1024 in
+// 1024).  A step of 1024^2 takes the same with 4 and 16 times the limit.
 #ifndef IMPEC_FOLD_READS
 #define IMPEC_FOLD_READS (1l << 20)
 #endif

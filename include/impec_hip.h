@@ -315,8 +315,10 @@ int impec_set_warmstart(impec_ctx *ctx, impec_cnn *net);
  * source, permeability and concentration, and read its fields and
  * diagnostics, with the usual calls (do not destroy it).  A member's fields
  * after impec_ensemble_step equal, bit for bit, those impec_step computes on
- * a context of the same parameters (mg_rows included); dt[k] is member k's
- * time step (no output-time clipping) and its[k] its CG iterations. */
+ * a context of the same parameters (mg_rows included) while eps lies above the
+ * rounding floor (last_relres_floor); below it both end at that floor, after
+ * other restarts.  dt[k] is member k's time step (no output-time clipping) and
+ * its[k] its CG iterations. */
 typedef struct impec_ensemble impec_ensemble;
 int impec_ensemble_create(const impec_params *members, int count, impec_ensemble **out);
 int impec_ensemble_destroy(impec_ensemble *e);
