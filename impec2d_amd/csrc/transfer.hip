@@ -6,12 +6,13 @@
 // packed into the other half.  Nothing of the context is written.  The link takes
 // 57 GB/s, one thread copies into fresh pages at 10-14; a pageable 2-D copy moves
 // 3.2 GB/s here (135 MB in 41 ms; the velocity of 4096^2 cells, interleaved by one
-// thread, in 143 ms).  c and v of 64^2 cells take 14 and 15 us, of 1024^2 0.31 and
+// thread, in 143 ms).  c and v of 64^2 cells take 14 and 15 us, of 1024^2 0.32 and
 // 0.47 ms, of 4096^2 2.7 and 5.3 ms; packed into device memory and copied from
 // there 30 and 52 us, 0.39 and 0.56 ms, 3.0 and 5.7 ms.  Where there is no pinned
 // memory to be had, or none free, the pageable copies serve.
 #include "impec_device.h"
 #include <atomic>
+#include <condition_variable>
 #include <mutex>
 #include <new>
 #include <thread>
@@ -89,9 +90,14 @@ void stage_give(const Stage &s) {
 }
 
 // Slices of consecutive chunks copied by `n` threads, the caller among them:
-// start() hands out a chunk, finish() copies the caller's share and waits for
-// the others'.
+// copy() hands out a chunk, copies the caller's share and waits for the others'.
+// Between chunks the threads look for the next one SPINS times, about as long as
+// a chunk that is due takes, then sleep: where the caller copies slower than the
+// link brings chunks they hardly ever do.
 struct Copiers {
+    static constexpr int SPINS = 64;
+    std::mutex m;
+    std::condition_variable go;
     std::atomic<int> chunk{0}, left{0};
     std::atomic<bool> stop{false};
     char *dst = nullptr;
@@ -107,9 +113,14 @@ struct Copiers {
     void worker(int k) {
         int seen = 0;
         for (;;) {
-            while (chunk.load(std::memory_order_acquire) == seen) {
+            for (int spin = 0; chunk.load(std::memory_order_acquire) == seen; spin++) {
                 if (stop.load(std::memory_order_acquire)) return;
-                std::this_thread::yield();
+                if (spin < SPINS) {
+                    std::this_thread::yield();
+                } else {
+                    std::unique_lock<std::mutex> l(m);
+                    go.wait(l, [&] { return chunk.load() != seen || stop.load(); });
+                }
             }
             seen++;
             share(k);
@@ -133,12 +144,20 @@ struct Copiers {
         src = s;
         bytes = b;
         left.store(n - 1, std::memory_order_relaxed);
-        chunk.fetch_add(1, std::memory_order_release);
+        {
+            std::lock_guard<std::mutex> l(m);
+            chunk.fetch_add(1, std::memory_order_release);
+        }
+        go.notify_all();
         share(0);
         while (left.load(std::memory_order_acquire) > 0) std::this_thread::yield();
     }
     ~Copiers() {
-        stop.store(true, std::memory_order_release);
+        {
+            std::lock_guard<std::mutex> l(m);
+            stop.store(true, std::memory_order_release);
+        }
+        go.notify_all();
         for (std::thread &t : threads) t.join();
     }
 };
@@ -179,7 +198,7 @@ static int get_chunks(impec_ctx *ctx, const Stage &st, double *dst, const double
         return IMPEC_OK;
     };
     const int nthreads = copy_threads(total * sizeof(double));
-    // the copying threads look for work in turn: not before the stream has come to it
+    // the copying threads start when the stream has come to the read
     if (nthreads > 1) IMPEC_HIP_CHECK(ctx, hipStreamSynchronize(ctx->stream));
     if (int e = queue(0)) return e;
     Copiers pool(nthreads);
