@@ -111,6 +111,31 @@ def test_source_split_bitexact(gpu_lib, profile, stype):
         assert abs(out_gpu - out_ref) <= 1e-14 * abs(out_ref)
 
 
+@pytest.mark.parametrize("wells", [1, 7, 8, 9, 1023, 1025, 4095, 4096, 4097])
+def test_outflux_of_many_wells(gpu_lib, wells):
+    """The outflux is summed over the wells in their order, bit for bit, up to 4096
+    of them (in LDS, eight at a time), and as a tree above (2^-53 times the number
+    of terms)."""
+    p = params(N1=70, N2=65, stype=1)
+    _say("outflux of wells", wells)
+    o, g = pair(p)
+    rng = np.random.default_rng(wells)
+    q = np.zeros(70 * 65)
+    cells = rng.permutation(q.size)[:wells]
+    q[cells] = rng.uniform(0.5, 2.0, wells) * np.where(np.arange(wells) % 3 < 2, -1.0, 1.0)
+    q = q.reshape(70, 65)
+    c = random_c(o, seed=wells)
+    g.set_source(q)
+    g.set_concentration(c)
+    for dt in (1e-3, 3e-2):
+        g.source_split(dt)
+        o.L.or_source_split(o.ctx, c, q, dt)
+    assert np.array_equal(g.get_concentration(), c)
+    got, want = g.stats().total_mass_outflux, o.total_mass_outflux
+    assert want > 0
+    assert got == want if wells <= 4096 else abs(got - want) < wells * 2.0 ** -53 * want
+
+
 @pytest.mark.parametrize("kw", [dict(dim_split=4), dict(dim_split=0), dict(dim_split=1), dict(dim_split=2),
                                 dict(dim_split=3), dict(dim_split=4, hyper=1), dict(dim_split=4, porosity=0.7),
                                 dict(dim_split=4, is_test=1), dict(dim_split=4, N1=21, N2=11),
