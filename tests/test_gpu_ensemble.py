@@ -130,6 +130,27 @@ def test_large_member_equal_single_context_bitwise(gpu_lib):
             assert np.array_equal(c_e, c_s)
 
 
+@pytest.mark.parametrize("precision", [0, 1])
+def test_members_around_the_folded_sums_limit(gpu_lib, precision):
+    """A single context folds the sums of its CG passes into their readers up to
+    576^2 cells, an ensemble never does: the members' equality holds the folded sums
+    to the finishing launches' bits on both sides of that size, and over levels of
+    several tiles."""
+    _say("ensemble around the folded sums' limit", precision)
+    specs = [(576, 576, "diag", 10.0, 0.5), (577, 576, "diag", 10.0, 0.5), (258, 509, "diag", 5.0, 0.5)]
+    ens, Ks = _make_ensemble(specs, precision=precision)
+    res = _ensemble_steps(ens, 2)
+    ens.close()
+    for k, (p, K) in enumerate(Ks):
+        _, _, single = _run_single(p, K, 2, precision=precision)
+        for s in range(2):
+            dts, its, fields_e = res[s][0], res[s][1], res[s][2][k]
+            dt_s, its_s, c_s, p_s, v_s = single[s]
+            assert its[k] == its_s and dts[k] == dt_s
+            for a, b in zip(fields_e, (c_s, p_s, v_s)):
+                assert np.array_equal(a, b)
+
+
 def test_members_with_eps_below_rounding_floor(gpu_lib):
     """eps = 1e-15 lies below the FP64 rounding floor of every member's
     system: a member's recursion can stall short of it.  The device-side loop
