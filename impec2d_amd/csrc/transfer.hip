@@ -70,7 +70,9 @@ bool stage_take(Stage &s) {
         stage_count++;
     }
     s.half[0] = nullptr;
-    if (hipHostMalloc((void **)&s.half[0], 2 * STAGE_BYTES, hipHostMallocPortable | hipHostMallocMapped) != hipSuccess ||
+    // coherent: a kernel writes it, and the host reads it when the event has passed
+    const unsigned flags = hipHostMallocPortable | hipHostMallocMapped | hipHostMallocCoherent;
+    if (hipHostMalloc((void **)&s.half[0], 2 * STAGE_BYTES, flags) != hipSuccess ||
         hipHostGetDevicePointer((void **)&s.dev[0], s.half[0], 0) != hipSuccess) {
         (void)hipGetLastError();
         if (s.half[0]) hipHostFree(s.half[0]);
